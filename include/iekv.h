@@ -206,6 +206,17 @@ int iekv_gather_rows_arrays(const iekv_pool* pool, int32_t first_array, int32_t 
                             int32_t block_size, const int32_t* block_table, int32_t context_len,
                             void* out, int64_t out_bytes, hipStream_t stream);
 
+/* The same gather with the block table in HOST memory: the entries the context
+ * uses are checked (IEKV_ERR_RANGE for one outside the pool) and travel in the
+ * launch's own kernel arguments, 2 * IEKV_INLINE_IDS blocks per launch (a longer
+ * table is gathered in consecutive launches), so no table upload precedes it.
+ * Replaces: the same reference lines as iekv_gather_rows_arrays, whose tables are
+ * host lists. */
+int iekv_gather_rows_arrays_ids(const iekv_pool* pool, int32_t first_array, int32_t n_arrays,
+                                int32_t block_size, const int32_t* block_table,
+                                int32_t context_len, void* out, int64_t out_bytes,
+                                hipStream_t stream);
+
 /* Most bytes of block images one direct host launch moves: offloads and
  * restores whose host range lies in one pinned allocation mapped for the device
  * are moved by the pack / unpack kernel itself (it writes or reads the host

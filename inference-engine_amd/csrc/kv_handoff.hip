@@ -448,7 +448,7 @@ kv_move_images(PoolView src, PoolView dst, const char* __restrict__ /*src_stage*
                                           group, n_arrays);
 }
 
-// Row kernels on either side of the handoff. A pool row is one token's
+// Row kernel of the prefill side. A pool row is one token's
 // H x D values of one array (tile_bytes / block_size bytes); row r of array a
 // lives at base(a) + r * row_bytes, i.e. slot r of the reference's [N*bs, H, D]
 // array. `lanes` lanes (a power of two, at most a wave) move one row with
@@ -459,12 +459,10 @@ kv_move_images(PoolView src, PoolView dst, const char* __restrict__ /*src_stage*
 // taking group w % chunks of array w / chunks; with `xcd`, position w is
 // XCD-grouped (kv_plan.h), so each of the 8 XCDs walks its own contiguous
 // share of arrays and rows. The scatter takes the XCD grouping from the order
-// of pool-writing launches, the gather from that of staging-writing ones.
-// Measured on MI355X, one launch per request, every layer or array at once
-// (GB/s, one box):
+// of pool-writing launches.
+// Measured on MI355X, one launch per request, every layer at once (GB/s, one box):
 //   Llama-3-8B shape (2 KiB rows): scatter 5,351 plain order -> 6,407 grouped,
-//     with non-temporal loads and stores (6,188 with ordinary stores); gather
-//     6,050 plain -> 5,698 grouped, so the gather stays in plain order;
+//     with non-temporal loads and stores (6,188 with ordinary stores);
 //   70B share, fp8 (1 KiB rows): scatter 5,677 plain, 5,566 grouped;
 //   one tensor-parallel rank of the 8B shape (256 B rows): scatter 4,880 plain,
 //     4,480 grouped, 5,091 with ordinary accesses.
@@ -472,7 +470,7 @@ kv_move_images(PoolView src, PoolView dst, const char* __restrict__ /*src_stage*
 constexpr int kWave = 64;
 constexpr int kRowU = 4;  // vectors per lane in flight: a 4 KiB row in one step
 // Stores of the scatter are non-temporal when the launch setting asks for
-// non-temporal accesses (the gather's always are then).
+// non-temporal accesses.
 #ifndef IEKV_SCATTER_NT_STORES
 #define IEKV_SCATTER_NT_STORES 1
 #endif
@@ -492,53 +490,6 @@ __device__ __forceinline__ void row_place(const RowShape& sh, int* array, int64_
   *first = static_cast<int64_t>(w % sh.chunks) * (kThreads / sh.lanes);
 }
 
-// Row `row` (< n) of this workgroup's share: addr(row, &src, &dst) gives its
-// addresses, or false to skip it (an id outside the pool). With WAVE_ROW (a
-// row spans the whole wave) the row index is made wave-uniform, so the id the
-// row's addresses depend on (a slot, a table entry) is read with one scalar load
-// instead of a vector load by all 64 lanes.
-template <bool WAVE_ROW, typename V, bool NTL, bool NTS, typename RowAddr>
-__device__ __forceinline__ void move_row_as(int64_t first, int32_t n, const RowShape& sh,
-                                            RowAddr addr) {
-  const int lanes = WAVE_ROW ? kWave : sh.lanes;
-  const int lane = threadIdx.x & (lanes - 1);
-  const int64_t row =
-      first + (WAVE_ROW ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave)
-                        : static_cast<int>(threadIdx.x) / lanes);
-  gptr<const V> s;
-  gptr<V> d;
-  if (row >= n || !addr(row, &s, &d)) return;
-  for (int e = lane; e < sh.row_vecs; e += kRowU * lanes) {
-    V v[kRowU];
-#pragma unroll
-    for (int u = 0; u < kRowU; ++u)
-      if (e + u * lanes < sh.row_vecs) v[u] = load_vec<V, NTL>(s + e + u * lanes);
-#pragma unroll
-    for (int u = 0; u < kRowU; ++u)
-      if (e + u * lanes < sh.row_vecs) store_vec<V, NTS>(d + e + u * lanes, v[u]);
-  }
-}
-
-// The gather reads its table entry with a scalar load when a row spans the
-// wave; the scatter keeps the vector load of its slot. Measured in alternating
-// processes on MI355X (two rounds each): the scalar load took the gather from
-// 6,388 / 6,385 to 6,664 / 6,713 GB/s on the 70B-shape share's 1 KiB rows and
-// from 6,096 / 6,100 to 6,148 / 6,151 on the 8B shape's 2 KiB rows; the scatter
-// read 5,322 / 5,342 with it against 5,592 / 6,156 without on the 1 KiB rows,
-// and tied on the 2 KiB rows.
-#ifndef IEKV_GATHER_UNIFORM_IDS
-#define IEKV_GATHER_UNIFORM_IDS 1
-#endif
-
-template <bool UNIFORM_IDS, typename V, bool NTL, bool NTS, typename RowAddr>
-__device__ __forceinline__ void move_row(int64_t first, int32_t n, const RowShape& sh,
-                                         RowAddr addr) {
-  if (UNIFORM_IDS && sh.lanes == kWave)
-    move_row_as<true, V, NTL, NTS>(first, n, sh, addr);
-  else
-    move_row_as<false, V, NTL, NTS>(first, n, sh, addr);
-}
-
 // The scatter loads a row's first vectors before it reads the row's slot, so
 // the two memory latencies overlap instead of adding up. Measured in five
 // rounds of alternating processes on MI355X: the 70B-shape share's write_kv
@@ -547,21 +498,15 @@ __device__ __forceinline__ void move_row(int64_t first, int32_t n, const RowShap
 // shape both orders fell into the same two placement modes (5.2-5.4 and
 // 6.3-6.4 TB/s). Reading the slot with a scalar load as well measured 5,290 /
 // 5,337 on the 1 KiB rows, so it stays a vector load.
-#ifndef IEKV_SCATTER_LOAD_FIRST
-#define IEKV_SCATTER_LOAD_FIRST 1
-#endif
-
 // A row whose source address is known before its destination: the row's first
 // vectors are loaded before the destination id is read. src_of(row) gives the
 // source, dst_of(row, &d) the destination or false to skip the row.
-template <bool WAVE_ROW, typename V, bool NTL, bool NTS, typename Src, typename Dst>
+template <typename V, bool NTL, bool NTS, typename Src, typename Dst>
 __device__ __forceinline__ void move_row_load_first(int64_t first, int32_t n,
                                                     const RowShape& sh, Src src_of, Dst dst_of) {
-  const int lanes = WAVE_ROW ? kWave : sh.lanes;
+  const int lanes = sh.lanes;
   const int lane = threadIdx.x & (lanes - 1);
-  const int64_t row =
-      first + (WAVE_ROW ? __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave)
-                        : static_cast<int>(threadIdx.x) / lanes);
+  const int64_t row = first + static_cast<int>(threadIdx.x) / lanes;
   if (row >= n) return;
   const gptr<const V> s = src_of(row);
   V v[kRowU];
@@ -600,49 +545,98 @@ kv_scatter_rows(PoolView pool, int32_t layers, int32_t first_layer, int32_t n_la
   const int64_t row_bytes = static_cast<int64_t>(sh.row_vecs) * sizeof(V);
   const char* src = (is_v ? v : k) + l * layer_stride;
   char* dst = array_base(pool, (is_v ? layers : 0) + first_layer + l);
-  if (IEKV_SCATTER_LOAD_FIRST) {
-    auto src_of = [&](int64_t i) { return as_global<V>(src + i * row_bytes); };
-    auto dst_of = [&](int64_t i, gptr<V>* d) {
-      const int64_t slot = slots[i];
-      if (slot < 0 || slot >= pool_rows) return false;  // never address outside the pool
-      *d = as_global<V>(dst + slot * row_bytes);
-      return true;
-    };
-    move_row_load_first<false, V, NTL, NTS>(first, n, sh, src_of, dst_of);
-    return;
-  }
-  move_row<false, V, NTL, NTS>(
-      first, n, sh, [&](int64_t i, gptr<const V>* s, gptr<V>* d) {
-        const int64_t slot = slots[i];
-        if (slot < 0 || slot >= pool_rows) return false;  // never address outside the pool
-        *s = as_global<V>(src + i * row_bytes);
-        *d = as_global<V>(dst + slot * row_bytes);
-        return true;
-      });
+  auto src_of = [&](int64_t i) { return as_global<V>(src + i * row_bytes); };
+  auto dst_of = [&](int64_t i, gptr<V>* d) {
+    const int64_t slot = slots[i];
+    if (slot < 0 || slot >= pool_rows) return false;  // never address outside the pool
+    *d = as_global<V>(dst + slot * row_bytes);
+    return true;
+  };
+  move_row_load_first<V, NTL, NTS>(first, n, sh, src_of, dst_of);
 }
 
-// gather_context over arrays: out row j (j < n) of array first_array + y, at
-// out + y * out_stride + j * row_bytes, is row table[j / bs] * bs + j % bs of
-// that array.
-template <typename V, bool NTL, bool NTS>
+// gather_context over arrays: the context of array first_array + y is one run of
+// bytes, at out + y * out_stride, put together from whole blocks and the used part
+// of the last one; a block's rows are one run in the pool too. So the gather works
+// in vectors of that run, whatever the row size: vector e is vector e % tile_vecs
+// of block table[e / tile_vecs], and every lane of a workgroup has one, also where
+// a row is no power of two of vectors (moving row by row, with a power of two of
+// lanes each, left 14 of 64 lanes idle on 800-byte rows). A launch covers `vecs`
+// vectors in each of its arrays, kThreads * U per workgroup, `chunks` workgroups
+// per array. It is bound by HBM: scattered 32 KiB reads against streaming writes.
+struct GatherShape {
+  int32_t tile_vecs;   // vectors per block
+  int32_t vecs;        // vectors per array in this launch (host: fits int32)
+  int32_t chunks;      // workgroups per array
+  int32_t xcd;         // 1: XCD-grouped workgroup positions
+  int32_t groups;      // workgroups in the launch (chunks * arrays; read instead of gridDim)
+};
+
+// The table of one launch in device memory, or carried in its kernel arguments.
+struct DeviceTable {
+  const int32_t* __restrict__ ids;
+  __device__ __forceinline__ int32_t operator[](int i) const { return ids[i]; }
+};
+template <int W>
+struct InlineTable {
+  int32_t ids[W];
+  __device__ __forceinline__ int32_t operator[](int i) const { return ids[i]; }
+};
+
+// SPANS: a workgroup's vectors may lie in several blocks (kThreads * U does not
+// divide tile_vecs), so each lane finds its own; otherwise the block, and its
+// table entry, are the same for the whole workgroup and read with scalar loads.
+template <typename V, int U, bool NT, bool SPANS, typename Table>
+__device__ __forceinline__ void gather_share(const PoolView& pool, int32_t first_array,
+                                             const Table& table, char* out, int64_t out_stride,
+                                             const GatherShape& sh) {
+  const uint32_t w = sh.xcd ? iekv_plan::xcd_grouped(blockIdx.x, sh.groups) : blockIdx.x;
+  const uint32_t y = w / sh.chunks;
+  const uint32_t base = (w - y * sh.chunks) * (kThreads * U);
+  const uint32_t block0 = base / sh.tile_vecs;
+  const uint32_t offset0 = base - block0 * sh.tile_vecs;
+  const char* src = array_base(pool, first_array + y);
+  const gptr<V> d = as_global<V>(out + y * out_stride) + base;
+  const int64_t tile_bytes = static_cast<int64_t>(sh.tile_vecs) * sizeof(V);
+  const uint32_t t = threadIdx.x;
+  const uint32_t left = sh.vecs - base;   // > 0: the last workgroup may hold fewer
+  V v[U];
+  bool have[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    uint32_t o = offset0 + u * kThreads + t;
+    uint32_t block = block0;
+    if constexpr (SPANS) {
+      const uint32_t q = o / sh.tile_vecs;
+      block += q;
+      o -= q * sh.tile_vecs;
+    }
+    have[u] = u * kThreads + t < left;
+    if (have[u]) {
+      const int32_t id = table[block];
+      have[u] = id >= 0 && id < pool.num_blocks;   // never address outside the pool
+      if (have[u]) v[u] = load_vec<V, NT>(as_global<V>(src + id * tile_bytes) + o);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (have[u]) store_vec<V, NT>(d + u * kThreads + t, v[u]);
+}
+
+template <typename V, int U, bool NT, bool SPANS>
 __global__ void __launch_bounds__(kThreads)
-kv_gather_rows(PoolView pool, int32_t first_array, const int32_t* __restrict__ table,
-               int32_t bs, char* __restrict__ out, int64_t out_stride, int32_t n,
-               RowShape sh) {
-  int y;
-  int64_t first;
-  row_place(sh, &y, &first);
-  const int64_t row_bytes = static_cast<int64_t>(sh.row_vecs) * sizeof(V);
-  const char* base = array_base(pool, first_array + y);
-  char* dst = out + y * out_stride;
-  move_row<IEKV_GATHER_UNIFORM_IDS != 0, V, NTL, NTS>(
-      first, n, sh, [&](int64_t j, gptr<const V>* s, gptr<V>* d) {
-    const int32_t block = table[j / bs];
-    if (block < 0 || block >= pool.num_blocks) return false;
-    *s = as_global<V>(base + (static_cast<int64_t>(block) * bs + j % bs) * row_bytes);
-    *d = as_global<V>(dst + j * row_bytes);
-    return true;
-  });
+kv_gather_rows(PoolView pool, int32_t first_array, DeviceTable table, char* __restrict__ out,
+               int64_t out_stride, GatherShape sh) {
+  gather_share<V, U, NT, SPANS>(pool, first_array, table, out, out_stride, sh);
+}
+
+// The same with the table in the kernel arguments (host block tables): no upload
+// precedes the launch.
+template <typename V, int U, bool NT, bool SPANS, int W>
+__global__ void __launch_bounds__(kThreads)
+kv_gather_inline(PoolView pool, int32_t first_array, InlineTable<W> table,
+                 char* __restrict__ out, int64_t out_stride, GatherShape sh) {
+  gather_share<V, U, NT, SPANS>(pool, first_array, table, out, out_stride, sh);
 }
 
 // Block-id checks of iekv_check_ids, three launches in stream order: clear the
@@ -1313,6 +1307,138 @@ int launch_list(const iekv_pool* pool, const char* src_stage, char* dst_stage, I
                                    host);
   return launch_move<SP, DP>(sp, dp, src_stage, dst_stage, s, d, n_blocks, pool->tile_bytes,
                              pool->n_arrays, align, stream, chunk, nt, host);
+}
+
+// Vectors per lane of a gather workgroup: 4 KiB of 16-byte vectors per workgroup.
+// Measured on MI355X with 1, 2 and 4: 8B shape, 7,777 tokens 318 / 333 / 334 us
+// (6.41 TB/s at 1; row by row it took 354); 70B share, 8,000 tokens 418 / 444 / 413;
+// 1,000 tokens 43.6 / 44.0 / 45.6; 800-byte rows, 3,000 tokens 43.7 / 45.3 / 48.9.
+// XCD-grouped positions cost 3-12% everywhere at 1, so the gather keeps the plain
+// order of staging-writing launches.
+constexpr int kGatherU = 1;
+// Table entries one gather launch carries in its arguments: a short block for the
+// contexts of small requests, a long one for 8,192 tokens in 16-token blocks
+// (arguments cost the host per KiB, see InlineIds).
+constexpr int kSmallTable = 64;
+constexpr int kLongTable = 2 * IEKV_INLINE_IDS;
+
+// A gather's arguments, checked before anything is enqueued.
+int check_gather(const iekv_pool* pool, int32_t first_array, int32_t n_arrays,
+                 int32_t block_size, const int32_t* block_table, int32_t context_len,
+                 const void* out, int64_t out_bytes) {
+  int rc;
+  if ((rc = check_pool(pool, "source"))) return rc;
+  if (first_array < 0 || n_arrays <= 0 || first_array > pool->n_arrays - n_arrays)
+    return set_error(IEKV_ERR_INVALID, "arrays %d..%d out of range for %d arrays", first_array,
+                     first_array + n_arrays - 1, pool->n_arrays);
+  if (block_size <= 0 || pool->tile_bytes % block_size)
+    return set_error(IEKV_ERR_INVALID, "block_size %d does not divide the %lld-byte tile",
+                     block_size, static_cast<long long>(pool->tile_bytes));
+  if (context_len < 0)
+    return set_error(IEKV_ERR_INVALID, "context_len is negative (%d)", context_len);
+  if (context_len == 0) return IEKV_OK;
+  const int64_t out_stride = pool->tile_bytes / block_size * context_len;
+  if (n_arrays > 1 && out_stride > INT64_MAX / n_arrays)
+    return set_error(IEKV_ERR_INVALID, "output size overflows");
+  if ((rc = check_buffer(out, out_bytes, out_stride * n_arrays, "output"))) return rc;
+  if (!block_table) return set_error(IEKV_ERR_INVALID, "block_table is null");
+  return IEKV_OK;
+}
+
+// One launch of a checked gather: `vecs` vectors of V per array, out of the blocks
+// of table[0 ..] (device memory, or `count` host ids for the arguments).
+template <typename V, int U>
+int launch_gather_as(const iekv_pool* pool, int32_t first_array, GatherShape sh, IdList table,
+                     int32_t count, char* out, int64_t out_stride, hipStream_t stream) {
+  const bool nt = g_nontemporal.load() != 0;
+  const bool spans = sh.tile_vecs % (kThreads * U) != 0;
+  const PoolView view = view_of(pool);
+  const dim3 grid(static_cast<uint32_t>(sh.groups));
+  auto inlined = [&](auto words) {
+    constexpr int W = decltype(words)::value;
+    InlineTable<W> t{};
+    std::copy(table.ids, table.ids + count, t.ids);
+    auto go = [&](auto kernel) {
+      return dispatch(kernel, grid, stream, view, first_array, t, out, out_stride, sh);
+    };
+    if (nt) return spans ? go(kv_gather_inline<V, U, true, true, W>)
+                         : go(kv_gather_inline<V, U, true, false, W>);
+    return spans ? go(kv_gather_inline<V, U, false, true, W>)
+                 : go(kv_gather_inline<V, U, false, false, W>);
+  };
+  if (table.on_host)
+    return count <= kSmallTable ? inlined(std::integral_constant<int, kSmallTable>{})
+                                : inlined(std::integral_constant<int, kLongTable>{});
+  const DeviceTable t{table.ids};
+  auto go = [&](auto kernel) {
+    return dispatch(kernel, grid, stream, view, first_array, t, out, out_stride, sh);
+  };
+  if (nt) return spans ? go(kv_gather_rows<V, U, true, true>)
+                       : go(kv_gather_rows<V, U, true, false>);
+  return spans ? go(kv_gather_rows<V, U, false, true>) : go(kv_gather_rows<V, U, false, false>);
+}
+
+// A checked gather of context_len >= 1 rows of n_arrays arrays, in launches of as
+// many blocks as the table in the arguments holds (host tables) and as 32-bit
+// vector numbers reach.
+int launch_gather(const iekv_pool* pool, int32_t first_array, int32_t n_arrays,
+                  int32_t block_size, IdList table, int32_t context_len, char* out,
+                  hipStream_t stream) {
+  const int64_t row_bytes = pool->tile_bytes / block_size;
+  const int64_t out_stride = row_bytes * context_len;
+  // Vectors as wide as the pool's tiles, the output and the distance between its
+  // arrays' contexts allow.
+  int vec = std::min(pool->align, align_of_ptr(reinterpret_cast<uint64_t>(out)));
+  vec = std::min(vec, align_of_ptr(static_cast<uint64_t>(out_stride)));
+  const int64_t tile_vecs = pool->tile_bytes / vec;
+  const int64_t per_group = kThreads * (vec == 16 ? kGatherU : 4);
+  // per_group more than the last vector stays below 2^31 too.
+  int64_t blocks_per_launch = std::max<int64_t>(1, (INT32_MAX - 2 * per_group) / tile_vecs);
+  if (table.on_host) blocks_per_launch = std::min<int64_t>(blocks_per_launch, kLongTable);
+  const int64_t blocks = (static_cast<int64_t>(context_len) - 1) / block_size + 1;
+  const int64_t most = std::min(blocks, blocks_per_launch) * tile_vecs;
+  if ((most + per_group - 1) / per_group * n_arrays > kMaxGrid)
+    return set_error(IEKV_ERR_INVALID, "a context of %d rows in %d arrays exceeds one launch",
+                     context_len, n_arrays);
+  DeviceGuard guard(pool->device);
+  if (!guard.ok()) return guard.fail();
+  for (int64_t first = 0; first < blocks; first += blocks_per_launch) {
+    const int64_t count = std::min(blocks_per_launch, blocks - first);
+    const int64_t begin = first * pool->tile_bytes;
+    const int64_t end = std::min((first + count) * pool->tile_bytes, out_stride);
+    GatherShape sh;
+    sh.tile_vecs = static_cast<int32_t>(tile_vecs);
+    sh.vecs = static_cast<int32_t>((end - begin) / vec);
+    sh.chunks = static_cast<int32_t>((sh.vecs + per_group - 1) / per_group);
+    sh.xcd = (g_pack_order.load() & iekv_plan::kXcdGrouped) != 0 ? 1 : 0;
+    sh.groups = sh.chunks * n_arrays;
+    const IdList part = table.from(first);
+    const int32_t n = static_cast<int32_t>(count);
+    int rc;
+    switch (vec) {
+      case 16:
+        rc = launch_gather_as<u32x4, kGatherU>(pool, first_array, sh, part, n, out + begin,
+                                               out_stride, stream);
+        break;
+      case 8:
+        rc = launch_gather_as<u32x2, 4>(pool, first_array, sh, part, n, out + begin, out_stride,
+                                        stream);
+        break;
+      case 4:
+        rc = launch_gather_as<uint32_t, 4>(pool, first_array, sh, part, n, out + begin,
+                                           out_stride, stream);
+        break;
+      case 2:
+        rc = launch_gather_as<uint16_t, 4>(pool, first_array, sh, part, n, out + begin,
+                                           out_stride, stream);
+        break;
+      default:
+        rc = launch_gather_as<uint8_t, 4>(pool, first_array, sh, part, n, out + begin,
+                                          out_stride, stream);
+    }
+    if (rc) return rc;
+  }
+  return IEKV_OK;
 }
 
 // Restore pipeline shared by the iekv_restore* calls: chunk k of the blocks is
@@ -2716,47 +2842,24 @@ int iekv_write_slots(const iekv_pool* pool, int32_t layer, int32_t block_size, c
 int iekv_gather_rows_arrays(const iekv_pool* pool, int32_t first_array, int32_t n_arrays,
                             int32_t block_size, const int32_t* block_table, int32_t context_len,
                             void* out, int64_t out_bytes, hipStream_t stream) {
-  int rc;
-  if ((rc = check_pool(pool, "source"))) return rc;
-  if (first_array < 0 || n_arrays <= 0 || first_array > pool->n_arrays - n_arrays)
-    return set_error(IEKV_ERR_INVALID, "arrays %d..%d out of range for %d arrays", first_array,
-                     first_array + n_arrays - 1, pool->n_arrays);
-  if (block_size <= 0 || pool->tile_bytes % block_size)
-    return set_error(IEKV_ERR_INVALID, "block_size %d does not divide the %lld-byte tile",
-                     block_size, static_cast<long long>(pool->tile_bytes));
-  if (context_len < 0)
-    return set_error(IEKV_ERR_INVALID, "context_len is negative (%d)", context_len);
-  if (context_len == 0) return IEKV_OK;
-  const int64_t row_bytes = pool->tile_bytes / block_size;
-  const int64_t out_stride = row_bytes * context_len;
-  if (n_arrays > 1 && out_stride > INT64_MAX / n_arrays)
-    return set_error(IEKV_ERR_INVALID, "output size overflows");
-  if ((rc = check_buffer(out, out_bytes, out_stride * n_arrays, "output"))) return rc;
-  if (!block_table) return set_error(IEKV_ERR_INVALID, "block_table is null");
-  const int align = row_align(row_bytes, pool->align, {out});
-  const int vec = align >= 16 ? 16 : align;
-  RowShape sh;
-  uint32_t grid = 0;
-  if (!row_shape(row_bytes, vec, context_len, n_arrays,
-                 (g_pack_order.load() & iekv_plan::kXcdGrouped) != 0, &sh, &grid))
-    return set_error(IEKV_ERR_INVALID, "a context of %d rows in %d arrays exceeds one launch",
-                     context_len, n_arrays);
-  DeviceGuard guard(pool->device);
-  if (!guard.ok()) return guard.fail();
-  char* oc = static_cast<char*>(out);
-  const PoolView view = view_of(pool);
-  const bool nt = g_nontemporal.load() != 0;
-#define IEKV_GATHER(T)                                                                      \
-  (nt ? dispatch(kv_gather_rows<T, true, true>, dim3(grid), stream, view, first_array,      \
-                 block_table, block_size, oc, out_stride, context_len, sh)                  \
-      : dispatch(kv_gather_rows<T, false, false>, dim3(grid), stream, view, first_array,    \
-                 block_table, block_size, oc, out_stride, context_len, sh))
-  if (vec >= 16) return IEKV_GATHER(u32x4);
-  if (vec >= 8) return IEKV_GATHER(u32x2);
-  if (vec >= 4) return IEKV_GATHER(uint32_t);
-  if (vec >= 2) return IEKV_GATHER(uint16_t);
-  return IEKV_GATHER(uint8_t);
-#undef IEKV_GATHER
+  const int rc = check_gather(pool, first_array, n_arrays, block_size, block_table, context_len,
+                              out, out_bytes);
+  if (rc || context_len == 0) return rc;
+  return launch_gather(pool, first_array, n_arrays, block_size, {block_table, false},
+                       context_len, static_cast<char*>(out), stream);
+}
+
+int iekv_gather_rows_arrays_ids(const iekv_pool* pool, int32_t first_array, int32_t n_arrays,
+                                int32_t block_size, const int32_t* block_table,
+                                int32_t context_len, void* out, int64_t out_bytes,
+                                hipStream_t stream) {
+  int rc = check_gather(pool, first_array, n_arrays, block_size, block_table, context_len, out,
+                        out_bytes);
+  if (rc || context_len == 0) return rc;
+  const int32_t blocks = (context_len - 1) / block_size + 1;
+  if ((rc = check_host_range(block_table, blocks, pool->num_blocks, "context"))) return rc;
+  return launch_gather(pool, first_array, n_arrays, block_size, {block_table, true},
+                       context_len, static_cast<char*>(out), stream);
 }
 
 int iekv_gather_rows(const iekv_pool* pool, int32_t array, int32_t block_size,

@@ -63,6 +63,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                         c_int64, c_void_p, c_int32, c_void_p]),
     "iekv_gather_rows_arrays": (c_int, [c_void_p, c_int32, c_int32, c_int32, c_void_p, c_int32,
                                         c_void_p, c_int64, c_void_p]),
+    "iekv_gather_rows_arrays_ids": (c_int, [c_void_p, c_int32, c_int32, c_int32, c_void_p,
+                                            c_int32, c_void_p, c_int64, c_void_p]),
     "iekv_offload": (c_int, [c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_void_p, c_int64,
                              c_void_p, c_void_p]),
     "iekv_offload_static": (c_int, [c_void_p, c_void_p, c_int32, c_void_p, c_int64, c_void_p,

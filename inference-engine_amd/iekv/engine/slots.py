@@ -14,6 +14,8 @@ a sequence's context in every layer's K and V cache at once.
 """
 from __future__ import annotations
 
+from array import array as _ints
+
 import torch
 
 from .. import _native
@@ -56,6 +58,32 @@ def write_slots(pool: KVPool, layer: int, k: torch.Tensor, v: torch.Tensor, slot
                  vc.data_ptr(), st.data_ptr(), n, stream)
 
 
+def _context_table(pool: KVPool, block_table, context_len: int):
+    """The table entries a context uses, and the entry point that takes them: a device
+    int32 tensor as it is, host ids as an int32 array the library checks and carries in
+    its launch (no upload). IndexError for a table too short for the context."""
+    needed = -(-context_len // pool.block_size)
+    if isinstance(block_table, torch.Tensor):
+        table = block_table.to(dtype=torch.int32)
+        if table.numel() < needed:
+            raise IndexError(f"context of {context_len} needs {needed} blocks, table has "
+                             f"{table.numel()}")
+        return table[:needed].to(pool.device).contiguous(), "iekv_gather_rows_arrays"
+    if needed > len(block_table):
+        raise IndexError(f"context of {context_len} needs {needed} blocks, table has "
+                         f"{len(block_table)}")
+    used = list(block_table[:needed])
+    try:
+        return _ints("i", used), "iekv_gather_rows_arrays_ids"
+    except (TypeError, OverflowError):      # not 32-bit integers: refused as elsewhere
+        ids = pool.host_ids(used, what="context block")
+        return _ints("i", ids.tolist()), "iekv_gather_rows_arrays_ids"
+
+
+def _address(table) -> int:
+    return table.data_ptr() if isinstance(table, torch.Tensor) else table.buffer_info()[0]
+
+
 def gather_rows(pool: KVPool, array: int, block_table, context_len: int) -> torch.Tensor:
     """Rows ``0..context_len-1`` of a sequence in array ``array`` (K of layer l is l, V is L+l).
 
@@ -63,24 +91,11 @@ def gather_rows(pool: KVPool, array: int, block_table, context_len: int) -> torc
     IndexError when the table is too short for ``context_len`` (as the
     reference does) or holds a block outside the pool.
     """
-    bs = pool.block_size
-    needed = -(-context_len // bs)
-    if isinstance(block_table, torch.Tensor):
-        table = block_table.to(dtype=torch.int32)
-        if table.numel() < needed:
-            raise IndexError(f"context of {context_len} needs {needed} blocks, table has "
-                             f"{table.numel()}")
-        table = table[:needed].to(pool.device).contiguous()
-    else:
-        if needed > len(block_table):
-            raise IndexError(f"context of {context_len} needs {needed} blocks, table has "
-                             f"{len(block_table)}")
-        table = pool.block_ids(list(block_table[:needed]), what="context block")
+    table, fn = _context_table(pool, block_table, context_len)
     out = torch.empty((context_len, *pool.tile_shape[1:]), dtype=pool.dtype, device=pool.device)
-    stream = current_stream_handle(pool.device)
-    _native.call("iekv_gather_rows", pool.native.handle, array, bs, table.data_ptr(),
+    _native.call(fn, pool.native.handle, array, 1, pool.block_size, _address(table),
                  context_len, out.data_ptr(), out.numel() * out.element_size(),
-                 stream)
+                 current_stream_handle(pool.device))
     return out
 
 
@@ -128,23 +143,10 @@ def gather_rows_arrays(pool: KVPool, block_table, context_len: int, first_array:
     if first_array < 0 or n_arrays <= 0 or first_array + n_arrays > pool.n_arrays:
         raise IndexError(f"arrays {first_array}..{first_array + n_arrays - 1} out of range for "
                          f"{pool.n_arrays} arrays")
-    bs = pool.block_size
-    needed = -(-context_len // bs)
-    if isinstance(block_table, torch.Tensor):
-        table = block_table.to(dtype=torch.int32)
-        if table.numel() < needed:
-            raise IndexError(f"context of {context_len} needs {needed} blocks, table has "
-                             f"{table.numel()}")
-        table = table[:needed].to(pool.device).contiguous()
-    else:
-        if needed > len(block_table):
-            raise IndexError(f"context of {context_len} needs {needed} blocks, table has "
-                             f"{len(block_table)}")
-        table = pool.block_ids(list(block_table[:needed]), what="context block")
+    table, fn = _context_table(pool, block_table, context_len)
     out = torch.empty((n_arrays, context_len, *pool.tile_shape[1:]), dtype=pool.dtype,
                       device=pool.device)
-    stream = current_stream_handle(pool.device)
-    _native.call("iekv_gather_rows_arrays", pool.native.handle, first_array, n_arrays, bs,
-                 table.data_ptr(), context_len, out.data_ptr(), out.numel() * out.element_size(),
-                 stream)
+    _native.call(fn, pool.native.handle, first_array, n_arrays, pool.block_size,
+                 _address(table), context_len, out.data_ptr(),
+                 out.numel() * out.element_size(), current_stream_handle(pool.device))
     return out

@@ -248,3 +248,35 @@ def test_gather_takes_the_block_table_as_a_list_or_a_tensor(gpu):
             gather_rows(pool, 0, form[:3], context)
     oracle = gather_context(as_np(k[1]), table, context, bs)
     assert np.array_equal(as_np(want[1]), oracle.reshape(as_np(want[1]).shape))
+
+
+@pytest.mark.parametrize("bs,heads,dim,dtype", [
+    (2, 8, 128, torch.bfloat16),   # 256 vectors per block: one workgroup each
+    (1, 5, 80, torch.float16),     # 50 vectors per block: workgroups span blocks
+    (3, 1, 5, torch.float16),      # 30-byte blocks: the width follows the context's length
+])
+@pytest.mark.parametrize("blocks", [1, 64, 65, 512, 513, 1030])
+def test_host_tables_gather_like_device_tables_around_the_launch_limits(gpu, bs, heads, dim,
+                                                                        dtype, blocks):
+    """A list table rides in the launch's arguments (64 or 512 entries, longer ones in
+    several launches), a device table stays where it is: both read the rows the oracle
+    reads, with whole and partial last blocks."""
+    from iekv.engine.slots import gather_rows_arrays
+
+    n = 1040
+    k, v, pool = random_pool(n, bs, heads, dim, dtype, gpu, layers=2, seed=101)
+    table = [int(b) for b in np.random.default_rng(blocks).permutation(n)[:blocks]]
+    on_device = torch.tensor(table, dtype=torch.int32, device=gpu)
+    caches = [as_np(c) for c in k + v]
+    for context in {blocks * bs, (blocks - 1) * bs + 1}:
+        got = gather_rows_arrays(pool, table, context)
+        want = gather_rows_arrays(pool, on_device, context)
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+        for a, cache in enumerate(caches):
+            oracle = gather_context(cache, table, context, bs)
+            assert np.array_equal(as_np(got[a]).reshape(oracle.shape), oracle), (a, context)
+    for bad in (-1, n):
+        with pytest.raises(IndexError, match="context block id"):
+            gather_rows_arrays(pool, table[:-1] + [bad], blocks * bs)
+    with pytest.raises(TypeError):
+        gather_rows_arrays(pool, table[:-1] + [1.5], blocks * bs)
