@@ -195,6 +195,37 @@ int iekv_write_slots_layers(const iekv_pool* pool, int32_t first_layer, int32_t 
                             int64_t layer_stride, const int64_t* slots, int32_t n_tokens,
                             hipStream_t stream);
 
+/* Element types of rows and caches, for the scatters that cast. IEKV_TYPE_BYTES:
+ * rows that already hold the cache's bytes (row_type == cache_type means the same). */
+enum {
+  IEKV_TYPE_BYTES = 0,
+  IEKV_TYPE_F32 = 1,
+  IEKV_TYPE_F16 = 2,
+  IEKV_TYPE_BF16 = 3,
+  IEKV_TYPE_E4M3 = 4 /* fp8 e4m3 without infinities */
+};
+
+/* iekv_write_slots_layers for rows of row_type in a cache of cache_type (float32 to
+ * float16, bfloat16 or e4m3; float16 or bfloat16 to e4m3; any other pair of different
+ * types returns IEKV_ERR_INVALID): each element is rounded to nearest even on its way,
+ * so no cast pass precedes the call. Row i of layer l is at k + l * layer_stride +
+ * i * (row bytes in row_type). Values past the largest e4m3 value, and NaNs, become
+ * NaN.
+ * Replaces: `k.to(cache dtype)` and index_copy_ (ie/kernels/torch_backend.py:13-16). */
+int iekv_write_slots_cast(const iekv_pool* pool, int32_t first_layer, int32_t n_layers,
+                          int32_t block_size, const void* k, const void* v,
+                          int64_t layer_stride, const int64_t* slots, int32_t n_tokens,
+                          int32_t row_type, int32_t cache_type, hipStream_t stream);
+
+/* The same with the slots in HOST memory: checked (IEKV_ERR_RANGE for one outside the
+ * pool), then carried in the launches' own kernel arguments, IEKV_INLINE_IDS tokens per
+ * launch, so no upload precedes them.
+ * Replaces: the same reference lines, whose slot mappings are host lists. */
+int iekv_write_slots_cast_ids(const iekv_pool* pool, int32_t first_layer, int32_t n_layers,
+                              int32_t block_size, const void* k, const void* v,
+                              int64_t layer_stride, const int64_t* slots, int32_t n_tokens,
+                              int32_t row_type, int32_t cache_type, hipStream_t stream);
+
 /* gather_context for several arrays in one launch: out is [n_arrays][context_len]
  * [row] bytes (out_bytes checked); its slab y holds the context of array
  * first_array + y, row j = row block_table[j / block_size] * block_size +

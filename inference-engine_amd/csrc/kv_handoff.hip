@@ -448,111 +448,166 @@ kv_move_images(PoolView src, PoolView dst, const char* __restrict__ /*src_stage*
                                           group, n_arrays);
 }
 
-// Row kernel of the prefill side. A pool row is one token's
-// H x D values of one array (tile_bytes / block_size bytes); row r of array a
-// lives at base(a) + r * row_bytes, i.e. slot r of the reference's [N*bs, H, D]
-// array. `lanes` lanes (a power of two, at most a wave) move one row with
-// lane-contiguous vectors, so a workgroup moves kThreads / lanes consecutive
-// rows of one array, and short rows do not leave most of a wave idle; a lane
-// keeps up to U vectors of its row in flight before storing them.
-// A launch covers `chunks` groups of rows in each of its arrays, workgroup w
-// taking group w % chunks of array w / chunks; with `xcd`, position w is
-// XCD-grouped (kv_plan.h), so each of the 8 XCDs walks its own contiguous
-// share of arrays and rows. The scatter takes the XCD grouping from the order
-// of pool-writing launches.
-// Measured on MI355X, one launch per request, every layer at once (GB/s, one box):
-//   Llama-3-8B shape (2 KiB rows): scatter 5,351 plain order -> 6,407 grouped,
-//     with non-temporal loads and stores (6,188 with ordinary stores);
-//   70B share, fp8 (1 KiB rows): scatter 5,677 plain, 5,566 grouped;
-//   one tensor-parallel rank of the 8B shape (256 B rows): scatter 4,880 plain,
-//     4,480 grouped, 5,091 with ordinary accesses.
-// One row per lane group beat two to eight in flight on both shapes.
 constexpr int kWave = 64;
-constexpr int kRowU = 4;  // vectors per lane in flight: a 4 KiB row in one step
-// Stores of the scatter are non-temporal when the launch setting asks for
-// non-temporal accesses.
-#ifndef IEKV_SCATTER_NT_STORES
-#define IEKV_SCATTER_NT_STORES 1
-#endif
 
-struct RowShape {
-  int32_t row_vecs;  // vectors per row
-  int32_t lanes;     // lanes per row (a power of two dividing kWave)
-  int32_t chunks;    // groups of kThreads / lanes rows per array
-  int32_t xcd;       // 1: XCD-grouped workgroup positions
-  int32_t groups;    // workgroups in the launch (chunks * arrays; read instead of gridDim)
+// write_kv over layers, the prefill side. A pool row is one token's H x D values of
+// one array; row i of layer l of k (and of v), at k + l * layer_stride + i * (source
+// row bytes), lands in row slots[i] of K array first_layer + l (and of V array
+// layers + first_layer + l). Array index y of the launch is K of layer y for
+// y < n_layers, then V. A layer's rows are one run of bytes, so the scatter works in
+// vectors of that run, kThreads * U per workgroup, whatever the row size: a vector's
+// row is its number / row_vecs, and every lane has one (see the gather below).
+// The source vectors are loaded before the slots are read, so the two latencies
+// overlap (the 70B-shape share's 1 KiB rows ran at 6.13-6.30 TB/s that way, 5.47-5.57
+// with the slot read first).
+struct ScatterShape {
+  int32_t row_vecs;   // source vectors per row
+  int32_t vecs;       // source vectors per layer in this launch (host: fits int32)
+  int32_t chunks;     // workgroups per array
+  int32_t xcd;        // 1: XCD-grouped workgroup positions
+  int32_t groups;     // workgroups in the launch (chunks * arrays; read instead of gridDim)
 };
 
-// The (array index, first row) of this workgroup.
-__device__ __forceinline__ void row_place(const RowShape& sh, int* array, int64_t* first) {
-  const int w = sh.xcd ? iekv_plan::xcd_grouped(blockIdx.x, sh.groups) : blockIdx.x;
-  *array = w / sh.chunks;
-  *first = static_cast<int64_t>(w % sh.chunks) * (kThreads / sh.lanes);
-}
+// The slots of one launch in device memory, or carried in its kernel arguments.
+struct DeviceSlots {
+  const int64_t* __restrict__ slots;
+  __device__ __forceinline__ int64_t operator[](int i) const { return slots[i]; }
+};
+template <int W>
+struct InlineSlots {
+  int64_t slots[W];
+  __device__ __forceinline__ int64_t operator[](int i) const { return slots[i]; }
+};
 
-// The scatter loads a row's first vectors before it reads the row's slot, so
-// the two memory latencies overlap instead of adding up. Measured in five
-// rounds of alternating processes on MI355X: the 70B-shape share's write_kv
-// (1 KiB rows) read 6,126 / 5,376 / 6,302 / 6,292 / 6,293 GB/s against
-// 5,475 / 5,526 / 5,473 / 5,568 / 5,481 with the slot read first; on the 8B
-// shape both orders fell into the same two placement modes (5.2-5.4 and
-// 6.3-6.4 TB/s). Reading the slot with a scalar load as well measured 5,290 /
-// 5,337 on the 1 KiB rows, so it stays a vector load.
-// A row whose source address is known before its destination: the row's first
-// vectors are loaded before the destination id is read. src_of(row) gives the
-// source, dst_of(row, &d) the destination or false to skip the row.
-template <typename V, bool NTL, bool NTS, typename Src, typename Dst>
-__device__ __forceinline__ void move_row_load_first(int64_t first, int32_t n,
-                                                    const RowShape& sh, Src src_of, Dst dst_of) {
-  const int lanes = sh.lanes;
-  const int lane = threadIdx.x & (lanes - 1);
-  const int64_t row = first + static_cast<int>(threadIdx.x) / lanes;
-  if (row >= n) return;
-  const gptr<const V> s = src_of(row);
-  V v[kRowU];
-  int e = lane;
+// What happens to a vector between its load and its store. Bytes<V> moves it; the
+// casts round each element to the cache's type, to nearest even, so rows computed in
+// a wider type are written without a cast pass (which reads the wide rows, writes the
+// narrow ones and is followed by a launch that reads them again). A float past the
+// largest e4m3 value becomes its NaN; NaNs become the cache type's canonical one, the
+// sign kept for e4m3: bit for bit what torch's casts give.
+template <typename V>
+struct Bytes {
+  using Src = V;
+  using Dst = V;
+  static __device__ __forceinline__ V run(V v) { return v; }
+};
+
+struct FromF32 {
+  using Elem = uint32_t;
+  static __device__ __forceinline__ float value(uint32_t e) { return __builtin_bit_cast(float, e); }
+};
+struct FromF16 {
+  using Elem = uint16_t;
+  static __device__ __forceinline__ float value(uint32_t e) {
+    return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(e)));
+  }
+};
+struct FromBf16 {
+  using Elem = uint16_t;
+  static __device__ __forceinline__ float value(uint32_t e) {
+    return __builtin_bit_cast(float, e << 16);
+  }
+};
+struct ToF16 {
+  using Elem = uint16_t;
+  static __device__ __forceinline__ uint32_t code(float x) {
+    return __builtin_bit_cast(uint16_t, static_cast<_Float16>(x));
+  }
+};
+struct ToBf16 {
+  using Elem = uint16_t;
+  static __device__ __forceinline__ uint32_t code(float x) {
+    return x != x ? 0x7fc0u : __builtin_bit_cast(uint16_t, static_cast<__bf16>(x));
+  }
+};
+struct ToE4m3 {
+  using Elem = uint8_t;
+  static __device__ __forceinline__ uint32_t code(float x) {
+    const uint32_t sign = __builtin_bit_cast(uint32_t, x) >> 24 & 0x80u;
+    return x != x ? sign | 0x7fu
+                  : static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(x, x, 0, false)) & 0xffu;
+  }
+};
+
+template <int BYTES>
+using raw_bytes = std::conditional_t<
+    BYTES == 16, u32x4,
+    std::conditional_t<BYTES == 8, u32x2,
+                       std::conditional_t<BYTES == 4, uint32_t,
+                                          std::conditional_t<BYTES == 2, uint16_t, uint8_t>>>>;
+
+// N elements of From to N of To.
+template <typename From, typename To, int N>
+struct Cast {
+  using Src = raw_bytes<N * sizeof(typename From::Elem)>;
+  using Dst = raw_bytes<N * sizeof(typename To::Elem)>;
+  static __device__ __forceinline__ Dst run(Src v) {
+    typename From::Elem in[N];
+    typename To::Elem out[N];
+    __builtin_memcpy(in, &v, sizeof(in));
 #pragma unroll
-  for (int u = 0; u < kRowU; ++u)
-    if (e + u * lanes < sh.row_vecs) v[u] = load_vec<V, NTL>(s + e + u * lanes);
-  gptr<V> d;
-  if (!dst_of(row, &d)) return;
-  while (true) {
+    for (int i = 0; i < N; ++i)
+      out[i] = static_cast<typename To::Elem>(To::code(From::value(in[i])));
+    Dst d;
+    __builtin_memcpy(&d, out, sizeof(d));
+    return d;
+  }
+};
+
+template <typename Op, int U, bool NT, typename Slots>
+__device__ __forceinline__ void scatter_share(const PoolView& pool, int32_t layers,
+                                              int32_t first_layer, int32_t n_layers,
+                                              const char* k, const char* v, int64_t layer_stride,
+                                              const Slots& slots, int64_t pool_rows,
+                                              const ScatterShape& sh) {
+  using Src = typename Op::Src;
+  using Dst = typename Op::Dst;
+  const uint32_t w = sh.xcd ? iekv_plan::xcd_grouped(blockIdx.x, sh.groups) : blockIdx.x;
+  const uint32_t y = w / sh.chunks;
+  const uint32_t base = (w - y * sh.chunks) * (kThreads * U);
+  const uint32_t row0 = base / sh.row_vecs;
+  const uint32_t offset0 = base - row0 * sh.row_vecs;
+  const bool is_v = y >= static_cast<uint32_t>(n_layers);
+  const int32_t l = is_v ? y - n_layers : y;
+  const gptr<const Src> s = as_global<Src>((is_v ? v : k) + l * layer_stride) + base;
+  char* dst = array_base(pool, (is_v ? layers : 0) + first_layer + l);
+  const int64_t row_bytes = static_cast<int64_t>(sh.row_vecs) * sizeof(Dst);
+  const uint32_t t = threadIdx.x;
+  const uint32_t left = sh.vecs - base;   // > 0: the last workgroup may hold fewer
+  Src r[U];
 #pragma unroll
-    for (int u = 0; u < kRowU; ++u)
-      if (e + u * lanes < sh.row_vecs) store_vec<V, NTS>(d + e + u * lanes, v[u]);
-    e += kRowU * lanes;
-    if (e >= sh.row_vecs) break;
+  for (int u = 0; u < U; ++u)
+    if (u * kThreads + t < left) r[u] = load_vec<Src, NT>(s + u * kThreads + t);
 #pragma unroll
-    for (int u = 0; u < kRowU; ++u)
-      if (e + u * lanes < sh.row_vecs) v[u] = load_vec<V, NTL>(s + e + u * lanes);
+  for (int u = 0; u < U; ++u) {
+    if (u * kThreads + t >= left) continue;
+    const uint32_t o = offset0 + u * kThreads + t;
+    const uint32_t q = o / sh.row_vecs;
+    const int64_t slot = slots[row0 + q];
+    if (slot < 0 || slot >= pool_rows) continue;   // never address outside the pool
+    store_vec<Dst, NT>(as_global<Dst>(dst + slot * row_bytes) + (o - q * sh.row_vecs),
+                       Op::run(r[u]));
   }
 }
 
-// write_kv over layers: row i of layer l of k (and of v), at
-// k + l * layer_stride + i * row_bytes, lands in row slots[i] of K array
-// first_layer + l (and of V array layers + first_layer + l). Array index y of
-// the launch is K of layer y for y < n_layers, then V.
-template <typename V, bool NTL, bool NTS>
+template <typename Op, int U, bool NT>
 __global__ void __launch_bounds__(kThreads)
 kv_scatter_rows(PoolView pool, int32_t layers, int32_t first_layer, int32_t n_layers,
                 const char* __restrict__ k, const char* __restrict__ v, int64_t layer_stride,
-                const int64_t* __restrict__ slots, int32_t n, RowShape sh, int64_t pool_rows) {
-  int y;
-  int64_t first;
-  row_place(sh, &y, &first);
-  const bool is_v = y >= n_layers;
-  const int l = is_v ? y - n_layers : y;
-  const int64_t row_bytes = static_cast<int64_t>(sh.row_vecs) * sizeof(V);
-  const char* src = (is_v ? v : k) + l * layer_stride;
-  char* dst = array_base(pool, (is_v ? layers : 0) + first_layer + l);
-  auto src_of = [&](int64_t i) { return as_global<V>(src + i * row_bytes); };
-  auto dst_of = [&](int64_t i, gptr<V>* d) {
-    const int64_t slot = slots[i];
-    if (slot < 0 || slot >= pool_rows) return false;  // never address outside the pool
-    *d = as_global<V>(dst + slot * row_bytes);
-    return true;
-  };
-  move_row_load_first<V, NTL, NTS>(first, n, sh, src_of, dst_of);
+                DeviceSlots slots, int64_t pool_rows, ScatterShape sh) {
+  scatter_share<Op, U, NT>(pool, layers, first_layer, n_layers, k, v, layer_stride, slots,
+                           pool_rows, sh);
+}
+
+// The same with the slots in the kernel arguments (host slot lists): no upload
+// precedes the launch.
+template <typename Op, int U, bool NT, int W>
+__global__ void __launch_bounds__(kThreads)
+kv_scatter_inline(PoolView pool, int32_t layers, int32_t first_layer, int32_t n_layers,
+                  const char* __restrict__ k, const char* __restrict__ v, int64_t layer_stride,
+                  InlineSlots<W> slots, int64_t pool_rows, ScatterShape sh) {
+  scatter_share<Op, U, NT>(pool, layers, first_layer, n_layers, k, v, layer_stride, slots,
+                           pool_rows, sh);
 }
 
 // gather_context over arrays: the context of array first_array + y is one run of
@@ -966,33 +1021,6 @@ int launch_images(const iekv_pool* pool, const InlineImages& images, const int32
                   pool->n_arrays, n_blocks, pl.parts, pl.group, pl.order);
 }
 
-// The shape of a row launch over n rows in each of n_arrays arrays: lanes per
-// row (the smallest power of two with a vector of the row for every lane, at
-// most a wave), row groups per array, and the workgroup order. False when the
-// launch would exceed the dispatch limit.
-bool row_shape(int64_t row_bytes, int vec_bytes, int64_t n, int32_t n_arrays, bool xcd,
-               RowShape* sh, uint32_t* grid) {
-  sh->row_vecs = static_cast<int32_t>(row_bytes / vec_bytes);
-  sh->lanes = 1;
-  while (sh->lanes < kWave && sh->lanes < sh->row_vecs) sh->lanes <<= 1;
-  const int64_t per_group = kThreads / sh->lanes;
-  const int64_t chunks = (n + per_group - 1) / per_group;
-  if (chunks * n_arrays > kMaxGrid) return false;
-  sh->chunks = static_cast<int32_t>(chunks);
-  sh->xcd = xcd ? 1 : 0;
-  sh->groups = static_cast<int32_t>(chunks * n_arrays);
-  *grid = static_cast<uint32_t>(sh->groups);
-  return true;
-}
-
-int row_align(int64_t row_bytes, int pool_align, std::initializer_list<const void*> ptrs) {
-  int align = 16;
-  while (align > 1 && (row_bytes % align)) align >>= 1;
-  align = std::min(align, pool_align);
-  for (const void* p : ptrs) align = std::min(align, align_of_ptr(reinterpret_cast<uint64_t>(p)));
-  return align;
-}
-
 int check_pool(const iekv_pool* p, const char* what) {
   if (!p) return set_error(IEKV_ERR_INVALID, "%s pool is null", what);
   return IEKV_OK;
@@ -1307,6 +1335,194 @@ int launch_list(const iekv_pool* pool, const char* src_stage, char* dst_stage, I
                                    host);
   return launch_move<SP, DP>(sp, dp, src_stage, dst_stage, s, d, n_blocks, pool->tile_bytes,
                              pool->n_arrays, align, stream, chunk, nt, host);
+}
+
+// One scatter of rows (iekv_write_slots_*): where they come from, where they go, and
+// the types of the rows and the cache.
+struct RowWrite {
+  const iekv_pool* pool;
+  int32_t first_layer, n_layers, block_size;
+  const char* k;
+  const char* v;
+  int64_t layer_stride;
+  int32_t row_type, cache_type;
+};
+
+// The slots of a scatter: in device memory, or host slots (checked) for the arguments.
+struct SlotList {
+  const int64_t* slots;
+  bool on_host;
+};
+
+// Bytes of one element of a row type; 0 for a type that no cast knows.
+int type_bytes(int32_t type) {
+  switch (type) {
+    case IEKV_TYPE_F32: return 4;
+    case IEKV_TYPE_F16:
+    case IEKV_TYPE_BF16: return 2;
+    case IEKV_TYPE_E4M3: return 1;
+    default: return 0;
+  }
+}
+
+// Whether a scatter casts; rows of the cache's own type move as bytes.
+bool casts(const RowWrite& w) { return w.row_type != w.cache_type; }
+
+bool known_cast(int32_t from, int32_t to) {
+  if (to == IEKV_TYPE_F16 || to == IEKV_TYPE_BF16) return from == IEKV_TYPE_F32;
+  return to == IEKV_TYPE_E4M3 &&
+         (from == IEKV_TYPE_F32 || from == IEKV_TYPE_F16 || from == IEKV_TYPE_BF16);
+}
+
+// A scatter's arguments, checked before anything is enqueued.
+int check_write(const RowWrite& w, const int64_t* slots, int32_t n_tokens) {
+  int rc;
+  const iekv_pool* pool = w.pool;
+  if ((rc = check_pool(pool, "destination"))) return rc;
+  const int32_t layers = pool->n_arrays / 2;
+  if (pool->n_arrays % 2 || w.first_layer < 0 || w.n_layers <= 0 ||
+      w.first_layer > layers - w.n_layers)
+    return set_error(IEKV_ERR_INVALID, "layers %d..%d out of range for %d layers", w.first_layer,
+                     w.first_layer + w.n_layers - 1, layers);
+  if (w.block_size <= 0 || pool->tile_bytes % w.block_size)
+    return set_error(IEKV_ERR_INVALID, "block_size %d does not divide the %lld-byte tile",
+                     w.block_size, static_cast<long long>(pool->tile_bytes));
+  if (casts(w)) {
+    if (!known_cast(w.row_type, w.cache_type))
+      return set_error(IEKV_ERR_INVALID, "no cast from row type %d to cache type %d", w.row_type,
+                       w.cache_type);
+    const int size = type_bytes(w.cache_type);
+    if (pool->tile_bytes / w.block_size % size || pool->align < size)
+      return set_error(IEKV_ERR_INVALID, "the pool's rows do not hold whole %d-byte elements",
+                       size);
+  }
+  if (w.layer_stride < 0)
+    return set_error(IEKV_ERR_INVALID, "layer_stride is negative (%lld)",
+                     static_cast<long long>(w.layer_stride));
+  if (n_tokens < 0) return set_error(IEKV_ERR_INVALID, "n_tokens is negative (%d)", n_tokens);
+  if (n_tokens == 0) return IEKV_OK;
+  if (!w.k || !w.v || !slots) return set_error(IEKV_ERR_INVALID, "k, v or slots is null");
+  if (casts(w)) {
+    const int size = type_bytes(w.row_type);
+    if (reinterpret_cast<uint64_t>(w.k) % size || reinterpret_cast<uint64_t>(w.v) % size ||
+        w.layer_stride % size)
+      return set_error(IEKV_ERR_INVALID, "k, v or layer_stride is not aligned to %d-byte elements",
+                       size);
+  }
+  return IEKV_OK;
+}
+
+// Vectors per lane of a scatter workgroup with 16-byte source vectors: one, and four
+// where a cast leaves 4 bytes of each (float32 to e4m3), whose stores fill a quarter
+// of a cache line per wave and gain from being issued together. Measured on MI355X
+// with 1, 2 and 4 (us, XCD-grouped): 8B shape, 3,001 bfloat16 rows 127 / 145 / 137
+// (row by row: 146); the same rows from float32 202 / 204 / 212, 5.85 TB/s at 1 (cast
+// by torch first: 330); 70B share, 8,000 bfloat16 rows to e4m3 688 / 719 / 716 (torch
+// first: 1,083), 3,000 float32 rows to e4m3 477 / 442 / 404 (torch first: 580).
+constexpr int kScatterU = 1;
+template <typename Op>
+constexpr int kCastU = sizeof(typename Op::Dst) <= 4 ? 4 : 1;
+// Slots one scatter launch carries in its arguments: a decode step's, and a longer
+// block (arguments cost the host per KiB, see InlineIds).
+constexpr int kSmallSlots = 64;
+constexpr int kLongSlots = IEKV_INLINE_IDS;
+
+// Launches a checked scatter whose rows are `row_vecs` vectors of Op::Src, in as many
+// launches as the slots in the arguments (host slots) and 32-bit vector numbers need.
+template <typename Op, int U>
+int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t row_vecs,
+                    hipStream_t stream) {
+  const int64_t per_group = kThreads * U;
+  const int32_t layers = w.pool->n_arrays / 2;
+  // per_group more than the last vector stays below 2^31 too.
+  int64_t per_launch = std::max<int64_t>(1, (INT32_MAX - 2 * per_group) / row_vecs);
+  if (list.on_host) per_launch = std::min<int64_t>(per_launch, kLongSlots);
+  const int64_t most = std::min<int64_t>(n_tokens, per_launch) * row_vecs;
+  if ((most + per_group - 1) / per_group * 2 * w.n_layers > kMaxGrid)
+    return set_error(IEKV_ERR_INVALID, "%d tokens in %d layers exceed one launch", n_tokens,
+                     w.n_layers);
+  DeviceGuard guard(w.pool->device);
+  if (!guard.ok()) return guard.fail();
+  const bool nt = g_nontemporal.load() != 0;
+  const PoolView view = view_of(w.pool);
+  const int64_t pool_rows = w.pool->num_blocks * w.block_size;
+  for (int64_t first = 0; first < n_tokens; first += per_launch) {
+    const int32_t n = static_cast<int32_t>(std::min<int64_t>(per_launch, n_tokens - first));
+    ScatterShape sh;
+    sh.row_vecs = static_cast<int32_t>(row_vecs);
+    sh.vecs = static_cast<int32_t>(n * row_vecs);
+    sh.chunks = static_cast<int32_t>((sh.vecs + per_group - 1) / per_group);
+    sh.xcd = (g_order.load() & iekv_plan::kXcdGrouped) != 0 ? 1 : 0;
+    sh.groups = sh.chunks * 2 * w.n_layers;
+    const int64_t skip = first * row_vecs * static_cast<int64_t>(sizeof(typename Op::Src));
+    auto go = [&](auto kernel, const auto& slots) {
+      return dispatch(kernel, dim3(static_cast<uint32_t>(sh.groups)), stream, view, layers,
+                      w.first_layer, w.n_layers, w.k + skip, w.v + skip, w.layer_stride, slots,
+                      pool_rows, sh);
+    };
+    auto inlined = [&](auto words) {
+      constexpr int W = decltype(words)::value;
+      InlineSlots<W> slots{};
+      std::copy(list.slots + first, list.slots + first + n, slots.slots);
+      return nt ? go(kv_scatter_inline<Op, U, true, W>, slots)
+                : go(kv_scatter_inline<Op, U, false, W>, slots);
+    };
+    int rc;
+    if (!list.on_host) {
+      const DeviceSlots slots{list.slots + first};
+      rc = nt ? go(kv_scatter_rows<Op, U, true>, slots) : go(kv_scatter_rows<Op, U, false>, slots);
+    } else if (n <= kSmallSlots) {
+      rc = inlined(std::integral_constant<int, kSmallSlots>{});
+    } else {
+      rc = inlined(std::integral_constant<int, kLongSlots>{});
+    }
+    if (rc) return rc;
+  }
+  return IEKV_OK;
+}
+
+// A cast, 16 source bytes a lane where the rows allow it, else one element.
+template <typename From, typename To>
+int launch_cast(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t row_elems, int align,
+                hipStream_t stream) {
+  constexpr int kWide = 16 / sizeof(typename From::Elem);
+  using Wide = Cast<From, To, kWide>;
+  // Both rows hold whole vectors, and both sides' addresses are multiples of them.
+  if (align == 16 && row_elems % kWide == 0 &&
+      w.pool->align >= static_cast<int>(sizeof(typename Wide::Dst)))
+    return launch_write_as<Wide, kCastU<Wide>>(w, list, n_tokens, row_elems / kWide, stream);
+  return launch_write_as<Cast<From, To, 1>, 4>(w, list, n_tokens, row_elems, stream);
+}
+
+// A checked scatter of n_tokens >= 1 rows.
+int launch_write(const RowWrite& w, SlotList list, int32_t n_tokens, hipStream_t stream) {
+  const int64_t row_bytes = w.pool->tile_bytes / w.block_size;   // of the cache
+  // What divides both sources' addresses and the distance between layers.
+  int align = std::min(align_of_ptr(reinterpret_cast<uint64_t>(w.k)),
+                       align_of_ptr(reinterpret_cast<uint64_t>(w.v)));
+  if (w.layer_stride) align = std::min(align, align_of_ptr(static_cast<uint64_t>(w.layer_stride)));
+  if (casts(w)) {
+    const int64_t elems = row_bytes / type_bytes(w.cache_type);
+    if (w.cache_type == IEKV_TYPE_F16)
+      return launch_cast<FromF32, ToF16>(w, list, n_tokens, elems, align, stream);
+    if (w.cache_type == IEKV_TYPE_BF16)
+      return launch_cast<FromF32, ToBf16>(w, list, n_tokens, elems, align, stream);
+    if (w.row_type == IEKV_TYPE_F32)
+      return launch_cast<FromF32, ToE4m3>(w, list, n_tokens, elems, align, stream);
+    if (w.row_type == IEKV_TYPE_F16)
+      return launch_cast<FromF16, ToE4m3>(w, list, n_tokens, elems, align, stream);
+    return launch_cast<FromBf16, ToE4m3>(w, list, n_tokens, elems, align, stream);
+  }
+  align = std::min({align, w.pool->align, align_of_ptr(static_cast<uint64_t>(row_bytes))});
+  const int64_t row_vecs = row_bytes / align;
+  switch (align) {
+    case 16:
+      return launch_write_as<Bytes<u32x4>, kScatterU>(w, list, n_tokens, row_vecs, stream);
+    case 8: return launch_write_as<Bytes<u32x2>, 4>(w, list, n_tokens, row_vecs, stream);
+    case 4: return launch_write_as<Bytes<uint32_t>, 4>(w, list, n_tokens, row_vecs, stream);
+    case 2: return launch_write_as<Bytes<uint16_t>, 4>(w, list, n_tokens, row_vecs, stream);
+    default: return launch_write_as<Bytes<uint8_t>, 4>(w, list, n_tokens, row_vecs, stream);
+  }
 }
 
 // Vectors per lane of a gather workgroup: 4 KiB of 16-byte vectors per workgroup.
@@ -2786,52 +3002,35 @@ int iekv_write_slots_layers(const iekv_pool* pool, int32_t first_layer, int32_t 
                             int32_t block_size, const void* k, const void* v,
                             int64_t layer_stride, const int64_t* slots, int32_t n_tokens,
                             hipStream_t stream) {
-  int rc;
-  if ((rc = check_pool(pool, "destination"))) return rc;
-  const int32_t layers = pool->n_arrays / 2;
-  if (pool->n_arrays % 2 || first_layer < 0 || n_layers <= 0 ||
-      first_layer > layers - n_layers)
-    return set_error(IEKV_ERR_INVALID, "layers %d..%d out of range for %d layers", first_layer,
-                     first_layer + n_layers - 1, layers);
-  if (block_size <= 0 || pool->tile_bytes % block_size)
-    return set_error(IEKV_ERR_INVALID, "block_size %d does not divide the %lld-byte tile",
-                     block_size, static_cast<long long>(pool->tile_bytes));
-  if (layer_stride < 0)
-    return set_error(IEKV_ERR_INVALID, "layer_stride is negative (%lld)",
-                     static_cast<long long>(layer_stride));
-  if (n_tokens < 0) return set_error(IEKV_ERR_INVALID, "n_tokens is negative (%d)", n_tokens);
-  if (n_tokens == 0) return IEKV_OK;
-  if (!k || !v || !slots) return set_error(IEKV_ERR_INVALID, "k, v or slots is null");
-  const int64_t row_bytes = pool->tile_bytes / block_size;
-  const int align = std::min(row_align(row_bytes, pool->align, {k, v}),
-                             layer_stride ? align_of_ptr(static_cast<uint64_t>(layer_stride))
-                                          : 16);
-  RowShape sh;
-  uint32_t grid = 0;
-  const int vec = align >= 16 ? 16 : align;
-  if (!row_shape(row_bytes, vec, n_tokens, 2 * n_layers,
-                 (g_order.load() & iekv_plan::kXcdGrouped) != 0, &sh, &grid))
-    return set_error(IEKV_ERR_INVALID, "%d tokens in %d layers exceed one launch", n_tokens,
-                     n_layers);
-  DeviceGuard guard(pool->device);
-  if (!guard.ok()) return guard.fail();
-  const int64_t pool_rows = pool->num_blocks * block_size;
-  const char* kc = static_cast<const char*>(k);
-  const char* vc = static_cast<const char*>(v);
-  const PoolView view = view_of(pool);
-  const bool nt = g_nontemporal.load() != 0;
-  constexpr bool kNts = IEKV_SCATTER_NT_STORES != 0;
-#define IEKV_SCATTER(T)                                                                      \
-  (nt ? dispatch(kv_scatter_rows<T, true, kNts>, dim3(grid), stream, view, layers,          \
-                 first_layer, n_layers, kc, vc, layer_stride, slots, n_tokens, sh, pool_rows) \
-      : dispatch(kv_scatter_rows<T, false, false>, dim3(grid), stream, view, layers,         \
-                 first_layer, n_layers, kc, vc, layer_stride, slots, n_tokens, sh, pool_rows))
-  if (vec >= 16) return IEKV_SCATTER(u32x4);
-  if (vec >= 8) return IEKV_SCATTER(u32x2);
-  if (vec >= 4) return IEKV_SCATTER(uint32_t);
-  if (vec >= 2) return IEKV_SCATTER(uint16_t);
-  return IEKV_SCATTER(uint8_t);
-#undef IEKV_SCATTER
+  return iekv_write_slots_cast(pool, first_layer, n_layers, block_size, k, v, layer_stride, slots,
+                               n_tokens, IEKV_TYPE_BYTES, IEKV_TYPE_BYTES, stream);
+}
+
+int iekv_write_slots_cast(const iekv_pool* pool, int32_t first_layer, int32_t n_layers,
+                          int32_t block_size, const void* k, const void* v,
+                          int64_t layer_stride, const int64_t* slots, int32_t n_tokens,
+                          int32_t row_type, int32_t cache_type, hipStream_t stream) {
+  const RowWrite w{pool, first_layer, n_layers, block_size, static_cast<const char*>(k),
+                   static_cast<const char*>(v), layer_stride, row_type, cache_type};
+  const int rc = check_write(w, slots, n_tokens);
+  if (rc || n_tokens == 0) return rc;
+  return launch_write(w, {slots, false}, n_tokens, stream);
+}
+
+int iekv_write_slots_cast_ids(const iekv_pool* pool, int32_t first_layer, int32_t n_layers,
+                              int32_t block_size, const void* k, const void* v,
+                              int64_t layer_stride, const int64_t* slots, int32_t n_tokens,
+                              int32_t row_type, int32_t cache_type, hipStream_t stream) {
+  const RowWrite w{pool, first_layer, n_layers, block_size, static_cast<const char*>(k),
+                   static_cast<const char*>(v), layer_stride, row_type, cache_type};
+  const int rc = check_write(w, slots, n_tokens);
+  if (rc || n_tokens == 0) return rc;
+  const int64_t rows = pool->num_blocks * block_size;
+  for (int32_t i = 0; i < n_tokens; ++i)
+    if (slots[i] < 0 || slots[i] >= rows)
+      return set_error(IEKV_ERR_RANGE, "slot %lld out of range for a pool of %lld slots",
+                       static_cast<long long>(slots[i]), static_cast<long long>(rows));
+  return launch_write(w, {slots, true}, n_tokens, stream);
 }
 
 int iekv_write_slots(const iekv_pool* pool, int32_t layer, int32_t block_size, const void* k,

@@ -29,6 +29,12 @@ IEKV_ERR_CAPACITY = -3
 IEKV_ERR_RANGE = -4      # a host block id outside its pool
 IEKV_ERR_IDS = -5        # host ids that conflict (a destination twice; overlap within a pool)
 IEKV_ERR_TIMEOUT = -6    # iekv_queue_wait: the requests did not finish in time
+# Element types of iekv_write_slots_cast.
+IEKV_TYPE_BYTES = 0
+IEKV_TYPE_F32 = 1
+IEKV_TYPE_F16 = 2
+IEKV_TYPE_BF16 = 3
+IEKV_TYPE_E4M3 = 4
 # Bits iekv_check_ids writes to its status word.
 IEKV_IDS_SRC_RANGE = 1
 IEKV_IDS_DST_RANGE = 2
@@ -61,6 +67,11 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                  c_int64, c_void_p]),
     "iekv_write_slots_layers": (c_int, [c_void_p, c_int32, c_int32, c_int32, c_void_p, c_void_p,
                                         c_int64, c_void_p, c_int32, c_void_p]),
+    "iekv_write_slots_cast": (c_int, [c_void_p, c_int32, c_int32, c_int32, c_void_p, c_void_p,
+                                      c_int64, c_void_p, c_int32, c_int32, c_int32, c_void_p]),
+    "iekv_write_slots_cast_ids": (c_int, [c_void_p, c_int32, c_int32, c_int32, c_void_p,
+                                          c_void_p, c_int64, c_void_p, c_int32, c_int32,
+                                          c_int32, c_void_p]),
     "iekv_gather_rows_arrays": (c_int, [c_void_p, c_int32, c_int32, c_int32, c_void_p, c_int32,
                                         c_void_p, c_int64, c_void_p]),
     "iekv_gather_rows_arrays_ids": (c_int, [c_void_p, c_int32, c_int32, c_int32, c_void_p,

@@ -16,26 +16,80 @@ from __future__ import annotations
 
 from array import array as _ints
 
+import numpy as np
 import torch
 
 from .. import _native
 from .pools import KVPool, current_stream_handle
 
 
-def _device_slots(slots, device: torch.device) -> torch.Tensor:
+# Longest host slot list the library carries in its launches' arguments (IEKV_INLINE_IDS
+# tokens each): two launches. Longer lists are uploaded once.
+HOST_SLOTS_MAX = 2 * _native.INLINE_IDS
+
+_TYPES = {torch.float32: _native.IEKV_TYPE_F32, torch.float16: _native.IEKV_TYPE_F16,
+          torch.bfloat16: _native.IEKV_TYPE_BF16, torch.float8_e4m3fn: _native.IEKV_TYPE_E4M3}
+# (row type, cache type) pairs iekv_write_slots_cast rounds on the way.
+_CASTS = {(torch.float32, torch.float16), (torch.float32, torch.bfloat16),
+          (torch.float32, torch.float8_e4m3fn), (torch.float16, torch.float8_e4m3fn),
+          (torch.bfloat16, torch.float8_e4m3fn)}
+
+
+def _slots(pool: KVPool, slots):
+    """The slots of a call as the library takes them, and the entry point that does: a
+    device int64 tensor, or a short host list as an int64 array that the library checks
+    and carries in its launch. Host slots outside the pool raise IndexError."""
     if isinstance(slots, torch.Tensor):
-        t = slots.to(device=device, dtype=torch.int64)
-    else:
-        t = torch.as_tensor(slots, dtype=torch.int64, device=device)
-    return t.contiguous()
+        t = slots.to(device=pool.device, dtype=torch.int64)
+        return t.contiguous(), "iekv_write_slots_cast"
+    rows = pool.num_blocks * pool.block_size
+    try:
+        host = _ints("q", slots if type(slots) in (list, tuple) else list(slots))
+    except (TypeError, OverflowError):      # not 64-bit integers
+        bad = [s for s in slots if not 0 <= int(s) < rows]
+        if bad:
+            raise IndexError(f"slot {bad[0]} out of range for a pool of {rows} slots")
+        t = torch.as_tensor(slots, dtype=torch.int64, device=pool.device)
+        return t.contiguous(), "iekv_write_slots_cast"
+    if len(host) <= HOST_SLOTS_MAX:
+        return host, "iekv_write_slots_cast_ids"
+    checked = np.frombuffer(host, dtype=np.int64)
+    if checked.min() < 0 or checked.max() >= rows:
+        bad = checked[(checked < 0) | (checked >= rows)][0]
+        raise IndexError(f"slot {bad} out of range for a pool of {rows} slots")
+    t = torch.from_numpy(checked).pin_memory().to(pool.device, non_blocking=True)
+    return t, "iekv_write_slots_cast"
+
+
+def _rows(pool: KVPool, k: torch.Tensor, v: torch.Tensor):
+    """K and V rows as the library reads them, and the types of the rows and the cache:
+    contiguous rows in a wider type that it can round itself as they are, others cast
+    first (the cast also makes them contiguous)."""
+    if k.dtype == v.dtype and (k.dtype, pool.dtype) in _CASTS and \
+            k.device == v.device == pool.device and not (k.is_neg() or v.is_neg()) and \
+            k.is_contiguous() and v.is_contiguous():
+        return k, v, _TYPES[k.dtype], _TYPES[pool.dtype]
+    return (k.to(device=pool.device, dtype=pool.dtype).contiguous(),
+            v.to(device=pool.device, dtype=pool.dtype).contiguous(),
+            _native.IEKV_TYPE_BYTES, _native.IEKV_TYPE_BYTES)
+
+
+def _write(pool: KVPool, first_layer: int, n_layers: int, n: int, k: torch.Tensor,
+           v: torch.Tensor, slots) -> None:
+    where, fn = _slots(pool, slots)
+    kc, vc, row_type, cache_type = _rows(pool, k, v)
+    stride = kc.numel() // n_layers * kc.element_size() if n_layers > 1 else 0
+    _native.call(fn, pool.native.handle, first_layer, n_layers, pool.block_size, kc.data_ptr(),
+                 vc.data_ptr(), stride, _address(where), n, row_type, cache_type,
+                 current_stream_handle(pool.device))
 
 
 def write_slots(pool: KVPool, layer: int, k: torch.Tensor, v: torch.Tensor, slots) -> None:
     """Scatter rows ``k[i]``, ``v[i]`` ([n, H, D]) into slot ``slots[i]`` of ``layer``.
 
-    The rows are cast to the cache dtype first (as ``index_copy_`` of
-    ``k.to(cache dtype)`` does); slots are range-checked on the host when given
-    as a list.
+    The rows are cast to the cache dtype (as ``index_copy_`` of
+    ``k.to(cache dtype)`` does), on their way where the library has the cast;
+    slots are range-checked on the host when given as a list.
     """
     n = k.shape[0]
     if v.shape[0] != n or len(slots) != n:
@@ -45,17 +99,7 @@ def write_slots(pool: KVPool, layer: int, k: torch.Tensor, v: torch.Tensor, slot
                          f"{pool.tile_shape[1:]}")
     if not 0 <= layer < pool.num_layers:
         raise IndexError(f"layer {layer} out of range for {pool.num_layers} layers")
-    if not isinstance(slots, torch.Tensor):
-        rows = pool.num_blocks * pool.block_size
-        bad = [s for s in slots if not 0 <= int(s) < rows]
-        if bad:
-            raise IndexError(f"slot {bad[0]} out of range for a pool of {rows} slots")
-    kc = k.to(device=pool.device, dtype=pool.dtype).contiguous()
-    vc = v.to(device=pool.device, dtype=pool.dtype).contiguous()
-    st = _device_slots(slots, pool.device)
-    stream = current_stream_handle(pool.device)
-    _native.call("iekv_write_slots", pool.native.handle, layer, pool.block_size, kc.data_ptr(),
-                 vc.data_ptr(), st.data_ptr(), n, stream)
+    _write(pool, layer, 1, n, k, v, slots)
 
 
 def _context_table(pool: KVPool, block_table, context_len: int):
@@ -99,14 +143,6 @@ def gather_rows(pool: KVPool, array: int, block_table, context_len: int) -> torc
     return out
 
 
-def _check_slots(pool: KVPool, slots) -> None:
-    if not isinstance(slots, torch.Tensor):
-        rows = pool.num_blocks * pool.block_size
-        bad = [s for s in slots if not 0 <= int(s) < rows]
-        if bad:
-            raise IndexError(f"slot {bad[0]} out of range for a pool of {rows} slots")
-
-
 def write_slots_layers(pool: KVPool, k: torch.Tensor, v: torch.Tensor, slots,
                        first_layer: int = 0) -> None:
     """Scatter ``k[l, i]``, ``v[l, i]`` ([n_layers, n, H, D]) into slot ``slots[i]`` of
@@ -123,15 +159,7 @@ def write_slots_layers(pool: KVPool, k: torch.Tensor, v: torch.Tensor, slots,
     if first_layer < 0 or first_layer + n_layers > pool.num_layers:
         raise IndexError(f"layers {first_layer}..{first_layer + n_layers - 1} out of range for "
                          f"{pool.num_layers} layers")
-    _check_slots(pool, slots)
-    kc = k.to(device=pool.device, dtype=pool.dtype).contiguous()
-    vc = v.to(device=pool.device, dtype=pool.dtype).contiguous()
-    st = _device_slots(slots, pool.device)
-    stride = n * kc.shape[2] * kc.shape[3] * kc.element_size()
-    stream = current_stream_handle(pool.device)
-    _native.call("iekv_write_slots_layers", pool.native.handle, first_layer, n_layers,
-                 pool.block_size, kc.data_ptr(), vc.data_ptr(), stride, st.data_ptr(), n,
-                 stream)
+    _write(pool, first_layer, n_layers, n, k, v, slots)
 
 
 def gather_rows_arrays(pool: KVPool, block_table, context_len: int, first_array: int = 0,

@@ -280,3 +280,54 @@ def test_host_tables_gather_like_device_tables_around_the_launch_limits(gpu, bs,
             gather_rows_arrays(pool, table[:-1] + [bad], blocks * bs)
     with pytest.raises(TypeError):
         gather_rows_arrays(pool, table[:-1] + [1.5], blocks * bs)
+
+
+@pytest.mark.parametrize("bs,heads,dim", [
+    (4, 8, 128),    # 1,024-element rows: 16-byte vectors
+    (2, 5, 80),     # rows of 100 and 25 source vectors: workgroups span rows
+    (3, 1, 6),      # rows that hold no whole 16-byte vector: one element per lane
+])
+@pytest.mark.parametrize("row_dtype,cache_dtype", [
+    (torch.float32, torch.float16), (torch.float32, torch.bfloat16),
+    (torch.float32, torch.float8_e4m3fn), (torch.float16, torch.float8_e4m3fn),
+    (torch.bfloat16, torch.float8_e4m3fn), (torch.float16, torch.float16),
+    (torch.float16, torch.float32),          # a pair torch casts first
+], ids=str)
+def test_rows_of_another_type_are_written_as_their_casts(gpu, bs, heads, dim, row_dtype,
+                                                         cache_dtype):
+    """Rows rounded on their way to the cache equal index_copy_ of k.to(cache dtype), NaNs,
+    infinities, overflows, ties and denormals included; slots as a list that one launch's
+    arguments hold, one that takes a longer block or two launches, one that is uploaded,
+    and a device tensor; aligned and odd row addresses."""
+    from iekv.engine.slots import write_slots, write_slots_layers
+
+    n_blocks = 700 // bs
+    rows_in_pool = n_blocks * bs
+    special = torch.tensor([0.0, -0.0, 1e-45, -3e-8, 6e-5, 447.9, 448.0, 456.0, 464.0, 464.1,
+                            480.0, -500.0, 65504.0, 65520.0, 1e30, float("inf"), -float("inf"),
+                            float("nan"), -float("nan"), 1.00390625, 0.0625 * 1.0625])
+    for n in (1, 64, 65, 256, 257, 512, 513):
+        k, v, pool = random_pool(n_blocks, bs, heads, dim, cache_dtype, gpu, layers=3, seed=n)
+        want = [c.clone() for c in k + v]
+        gen = torch.Generator(gpu).manual_seed(200 + n)
+        total = 2 * 2 * n * heads * dim
+        flat = torch.randn(total + 1, device=gpu, generator=gen) * 100
+        at = torch.randint(0, total, (total // 4 + 1,), device=gpu, generator=gen)
+        flat[at] = special.to(gpu)[torch.randint(0, special.numel(), at.shape, device=gpu,
+                                                 generator=gen)]
+        odd = n % 2                                 # odd: rows start one element in
+        rows = flat.to(row_dtype)[odd:odd + total].view(2, 2, n, heads, dim)
+        slots = [int(s) for s in np.random.default_rng(n).permutation(rows_in_pool)[:n]]
+        where = torch.tensor(slots, device=gpu)
+        write_slots_layers(pool, rows[0], rows[1], slots if n != 65 else where, first_layer=1)
+        for l in range(2):
+            want[1 + l].view(torch.uint8)[where] = rows[0, l].to(cache_dtype).view(torch.uint8)
+            want[4 + l].view(torch.uint8)[where] = rows[1, l].to(cache_dtype).view(torch.uint8)
+        write_slots(pool, 0, rows[1, 0], rows[0, 1], where if n != 65 else slots)
+        want[0].view(torch.uint8)[where] = rows[1, 0].to(cache_dtype).view(torch.uint8)
+        want[3].view(torch.uint8)[where] = rows[0, 1].to(cache_dtype).view(torch.uint8)
+        for a, (got, expected) in enumerate(zip(k + v, want)):
+            assert torch.equal(got.view(torch.uint8), expected.view(torch.uint8)), (n, a)
+        for bad in (-1, rows_in_pool):
+            with pytest.raises(IndexError, match=f"slot {bad} out of range"):
+                write_slots_layers(pool, rows[0], rows[1], slots[:-1] + [bad])
