@@ -1220,12 +1220,13 @@ int check_host_range(const int32_t* host_ids, int32_t n, int64_t num_blocks, con
 
 // IEKV_ERR_IDS unless the n ids at v are distinct.
 int check_distinct(const int32_t* v, int32_t n, const char* what) {
-  std::vector<int32_t> sorted(v, v + n);
-  std::sort(sorted.begin(), sorted.end());
+  std::vector<uint64_t> key(n);   // ids in the high half
+  for (int32_t i = 0; i < n; ++i) key[i] = static_cast<uint64_t>(static_cast<uint32_t>(v[i])) << 32;
+  iekv_plan::sort_by_high_half(&key);
   for (int32_t i = 1; i < n; ++i)
-    if (sorted[i] == sorted[i - 1])
+    if (key[i] == key[i - 1])
       return set_error(IEKV_ERR_IDS, "%s block ids must be distinct (id %d given twice)", what,
-                       sorted[i]);
+                       static_cast<int32_t>(key[i] >> 32));
   return IEKV_OK;
 }
 
@@ -1240,7 +1241,7 @@ int order_pairs(const int32_t* src_ids, const int32_t* dst_ids, int32_t n, bool 
   for (int32_t i = 0; i < n; ++i)
     key[i] = (static_cast<uint64_t>(static_cast<uint32_t>(dst_ids[i])) << 32) |
              static_cast<uint32_t>(src_ids[i]);
-  std::sort(key.begin(), key.end());
+  iekv_plan::sort_by_high_half(&key);
   src_out->resize(n);
   dst_out->resize(n);
   int32_t* s = src_out->data();

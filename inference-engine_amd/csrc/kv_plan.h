@@ -289,6 +289,48 @@ inline bool plan_slots(int64_t staging_bytes, int64_t block_bytes, int32_t n_blo
   return *slot_blocks >= 1;
 }
 
+// Sorts keys by their high 32 bits, keeping the order of equal ones: counting sorts
+// of 8 bits at a time, as many as the largest high half has, and none for keys that
+// already ascend (tables off a fresh free list). Below kCountingSortMin keys a
+// comparison sort is as fast. Measured on one x86 core with new random keys of 12
+// bits each time, against std::sort: 32 keys 0.88 / 0.73 us, 64 0.65 / 1.68, 193
+// 1.16 / 6.27, 1,088 4.8 / 46.7.
+constexpr size_t kCountingSortMin = 64;
+
+inline void sort_by_high_half(std::vector<uint64_t>* keys) {
+  const size_t n = keys->size();
+  uint64_t most = 0;
+  bool ascending = true;
+  for (size_t i = 0; i < n; ++i) {
+    const uint64_t high = (*keys)[i] >> 32;
+    if (i > 0 && high < (*keys)[i - 1] >> 32) ascending = false;
+    if (high > most) most = high;
+  }
+  if (ascending) return;
+  if (n < kCountingSortMin) {
+    std::stable_sort(keys->begin(), keys->end(),
+                     [](uint64_t x, uint64_t y) { return x >> 32 < y >> 32; });
+    return;
+  }
+  constexpr int kBits = 8;
+  std::vector<uint64_t> other(n);
+  for (int shift = 0; shift < 32 && most >> shift; shift += kBits) {
+    uint32_t first[1 << kBits] = {};
+    const auto digit = [shift](uint64_t key) {
+      return (key >> 32 >> shift) & ((1u << kBits) - 1);
+    };
+    for (size_t i = 0; i < n; ++i) ++first[digit((*keys)[i])];
+    uint32_t at = 0;
+    for (uint32_t& f : first) {
+      const uint32_t count = f;
+      f = at;
+      at += count;
+    }
+    for (size_t i = 0; i < n; ++i) other[first[digit((*keys)[i])]++] = (*keys)[i];
+    keys->swap(other);
+  }
+}
+
 // A byte range [lo, hi) of owner 0 or 1 (one pool's array, say).
 struct Span {
   uint64_t lo, hi;

@@ -571,6 +571,30 @@ static void check_queue_claims() {
     EXPECT(queue_claim_ring(slots) >= 2 * slots * kQueueMaxClaims, "claim ring too small");
 }
 
+// sort_by_high_half against std::stable_sort, on either side of its counting sorts'
+// limits: few and many keys, one to three digits, repeats, and keys that ascend.
+void check_sort() {
+  uint64_t state = 88172645463325252ull;
+  const auto next = [&] {
+    state ^= state << 13;
+    state ^= state >> 7;
+    state ^= state << 17;
+    return state;
+  };
+  for (size_t n : {0, 1, 2, 63, 64, 65, 1088, 5000})
+    for (uint64_t most : {1ull, 2047ull, 2048ull, (1ull << 22) - 1, 1ull << 22, 2147483646ull})
+      for (bool ascending : {false, true}) {
+        std::vector<uint64_t> keys(n), want;
+        for (size_t i = 0; i < n; ++i) keys[i] = (next() % (most + 1)) << 32 | (next() >> 33);
+        if (ascending) std::sort(keys.begin(), keys.end());
+        want = keys;
+        std::stable_sort(want.begin(), want.end(),
+                         [](uint64_t x, uint64_t y) { return x >> 32 < y >> 32; });
+        sort_by_high_half(&keys);
+        EXPECT(keys == want, "sorted by the high half, equal ones in their order");
+      }
+}
+
 int main() {
   check_queue_claims();
   for (int grid = 1; grid <= 4096; ++grid) check_xcd_grouped(grid);
@@ -635,6 +659,7 @@ int main() {
   check_image_views();
   check_pieces_and_slots();
   check_launch_chunk();
+  check_sort();
 
   if (failures) {
     std::printf("%d failures\n", failures);

@@ -1131,6 +1131,53 @@ def test_a_request_list_moves_each_request_on_its_stream_with_its_event(gpu):
     assert dst.blocks_written == sum(sizes)
 
 
+@pytest.mark.parametrize("sizes", [[], [0, 0], [1], [2047, 1], [2047, 2], [5, 0, 300, 1, 77]],
+                         ids=str)
+@pytest.mark.parametrize("n_streams", [0, 1, 2, 3])
+def test_requests_without_events_move_together(gpu, sizes, n_streams):
+    """copy_requests without events merges a stream's requests into launches that carry up
+    to 2,048 pairs in all, or into one launch per stream: the same bytes as the oracle's
+    handoffs, in every form of the tables, and the same refusals before anything moves."""
+    from iekv.engine.copier import HipSlotCopier
+
+    n, bs = 2600, 2
+    sk, sv = allocate(n, bs, 2, 1, 8, torch.float16, gpu, seed=111)
+    dk, dv = allocate(n, bs, 2, 1, 8, torch.float16, gpu, seed=112)
+    src_o, dst_o = oracle_of(sk, sv, bs), oracle_of(dk, dv, bs)
+    src, dst = HipSlotCopier(sk, sv, bs), HipSlotCopier(dk, dv, bs)
+    rng = np.random.default_rng(len(sizes) + n_streams)
+    forms = [list, tuple, np.array] if n_streams == 2 else [list, tuple]
+    streams = [torch.cuda.Stream() for _ in range(n_streams)] or None
+    src_perm, dst_perm = rng.permutation(n).tolist(), rng.permutation(n).tolist()
+    tables, at = [], 0
+    for k, m in enumerate(sizes):
+        form = forms[k % len(forms)]
+        tables.append((form(src_perm[at:at + m]), form(dst_perm[at:at + m])))
+        at += m
+    tables = [(np.asarray(s, np.int64), np.asarray(d, np.int64)) if isinstance(s, np.ndarray)
+              else (s, d) for s, d in tables]
+    dst.copy_requests(src, tables, streams=streams)
+    for st in streams or []:
+        st.synchronize()
+    handoff(src_o, dst_o, [list(t[0]) for t in tables], [list(t[1]) for t in tables])
+    assert_pool_equals(dk, dv, dst_o)
+    assert src.blocks_read == dst.blocks_written == sum(sizes)
+    for bad, error, match in (
+            ([([1], [5]), ([2], [5])], ValueError, "must be distinct"),
+            ([([1], [n])], IndexError, "out of range"),
+            ([([-1], [1])], IndexError, "out of range"),
+            ([([1, 2], [3])], ValueError, "2 source blocks for 1"),
+            ([([1.5], [3])], TypeError, "integers"),
+            ([([1], [2**40])], IndexError, "out of range")):
+        with pytest.raises(error, match=match):
+            dst.copy_requests(src, bad, streams=streams)
+    with pytest.raises(ValueError, match="disjoint"):
+        src.copy_requests(src, [([1], [2]), ([2], [3])], streams=streams)
+    torch.cuda.synchronize()
+    assert_pool_equals(dk, dv, dst_o)
+    assert dst.blocks_written == sum(sizes)
+
+
 def test_short_python_tables_and_numpy_tables_move_the_same_bytes(gpu):
     """Short Python tables go to the library unconverted (it checks and orders the
     ids), NumPy arrays and long lists through the NumPy checks; both must move the
