@@ -492,6 +492,24 @@ int iekv_check_ids(const iekv_pool* src, const int32_t* src_ids, const iekv_pool
                    const int32_t* dst_ids, int32_t n_blocks, void* workspace,
                    int64_t workspace_bytes, int32_t* status, hipStream_t stream);
 
+/* Most ids, and most destination blocks, of a check that runs as one workgroup in
+ * one launch, and of iekv_copy_direct_checked. */
+#define IEKV_CHECK_ONE_LAUNCH_IDS 8192
+#define IEKV_CHECK_ONE_LAUNCH_BLOCKS 262144
+
+/* iekv_check_ids and iekv_copy_direct back to back, without waiting in between: the
+ * check writes both id lists to `checked` (device memory, 2 * n_blocks int32), as
+ * they are or, when any check fails, as ids outside the pools, and the copy reads
+ * them there, so a list that fails moves nothing. The call returns once the check's
+ * result is known, in *bits (IEKV_IDS_*, 0 = the copy is on its way); `status` is a
+ * word of pinned host memory the result arrives in, the caller's own until the call
+ * returns. Lists or pools over the limits above return IEKV_ERR_CAPACITY, a stream
+ * under capture IEKV_ERR_INVALID.
+ * No counterpart in the reference (its copier checks no id). */
+int iekv_copy_direct_checked(const iekv_pool* src, const iekv_pool* dst, const int32_t* src_ids,
+                             const int32_t* dst_ids, int32_t n_blocks, int32_t* checked,
+                             int32_t* status, hipStream_t stream, int32_t* bits);
+
 /* Current launch shape, for reporting. */
 int iekv_get_launch(int32_t* run_blocks, int32_t* unroll, int32_t* nontemporal,
                     int32_t* order, int32_t* pack_order, int32_t* chunk_bytes);

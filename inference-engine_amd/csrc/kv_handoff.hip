@@ -737,6 +737,75 @@ ids_probe(const int32_t* __restrict__ ids, int32_t n, int64_t num_blocks,
   if (bitmap && (bitmap[id >> 5] >> (id & 31)) & 1u) atomicOr(status, IEKV_IDS_OVERLAP);
 }
 
+// The same checks in one launch of one workgroup, for lists and pools whose bitmap fits
+// its LDS: three dependent launches of about 4 us each become one (a launch this small
+// is all latency). With `checked` not null it also writes both lists there, sources
+// then destinations, or -1 for every id when a check failed: a move that reads them
+// right behind on the stream then moves nothing (an id outside its pool is skipped),
+// so the host need not wait between the check and the move. *status may be pinned
+// host memory: it is written once, after the lists.
+constexpr int kCheckThreads = 1024;
+constexpr int kCheckPerThread = 8;
+constexpr int32_t kCheckIds = kCheckThreads * kCheckPerThread;
+constexpr int64_t kCheckBlocks = IEKV_CHECK_ONE_LAUNCH_BLOCKS;   // a 32 KiB bitmap
+static_assert(kCheckIds == IEKV_CHECK_ONE_LAUNCH_IDS, "the header states the limit");
+
+__global__ void __launch_bounds__(kCheckThreads)
+ids_check(const int32_t* __restrict__ src_ids, const int32_t* __restrict__ dst_ids, int32_t n,
+          int64_t src_blocks, int64_t dst_blocks, int32_t same_pool,
+          int32_t* __restrict__ checked, int32_t* __restrict__ status) {
+  extern __shared__ uint32_t bitmap[];   // (dst_blocks + 31) / 32 words
+  __shared__ int32_t s_bits;
+  const int t = threadIdx.x;
+  int32_t src[kCheckPerThread], dst[kCheckPerThread];
+#pragma unroll
+  for (int j = 0; j < kCheckPerThread; ++j) {
+    const int i = j * kCheckThreads + t;
+    src[j] = src_ids && i < n ? src_ids[i] : 0;
+    dst[j] = dst_ids && i < n ? dst_ids[i] : 0;
+  }
+  if (t == 0) s_bits = 0;
+  if (dst_ids)
+    for (int w = t; w < (dst_blocks + 31) / 32; w += kCheckThreads) bitmap[w] = 0u;
+  __syncthreads();
+  int32_t bits = 0;
+  if (dst_ids) {
+#pragma unroll
+    for (int j = 0; j < kCheckPerThread; ++j) {
+      if (j * kCheckThreads + t >= n) continue;
+      if (dst[j] < 0 || dst[j] >= dst_blocks) {
+        bits |= IEKV_IDS_DST_RANGE;
+        continue;
+      }
+      const uint32_t bit = 1u << (dst[j] & 31);
+      if (atomicOr(&bitmap[dst[j] >> 5], bit) & bit) bits |= IEKV_IDS_DST_REPEATED;
+    }
+  }
+  __syncthreads();
+  if (src_ids) {
+#pragma unroll
+    for (int j = 0; j < kCheckPerThread; ++j) {
+      if (j * kCheckThreads + t >= n) continue;
+      if (src[j] < 0 || src[j] >= src_blocks) bits |= IEKV_IDS_SRC_RANGE;
+      else if (same_pool && src[j] < dst_blocks && (bitmap[src[j] >> 5] >> (src[j] & 31)) & 1u)
+        bits |= IEKV_IDS_OVERLAP;
+    }
+  }
+  if (bits) atomicOr(&s_bits, bits);
+  __syncthreads();
+  const int32_t found = s_bits;
+  if (checked) {
+#pragma unroll
+    for (int j = 0; j < kCheckPerThread; ++j) {
+      const int i = j * kCheckThreads + t;
+      if (i >= n) continue;
+      checked[i] = found ? -1 : src[j];
+      checked[n + i] = found ? -1 : dst[j];
+    }
+  }
+  if (t == 0) __hip_atomic_store(status, found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The launch floor (iekv_noop): a kernel that does nothing, so its duration is
 // the cost of dispatching, running and retiring its workgroups alone.
 __global__ void __launch_bounds__(kThreads) kv_noop() {}
@@ -1336,6 +1405,24 @@ int launch_list(const iekv_pool* pool, const char* src_stage, char* dst_stage, I
                                    host);
   return launch_move<SP, DP>(sp, dp, src_stage, dst_stage, s, d, n_blocks, pool->tile_bytes,
                              pool->n_arrays, align, stream, chunk, nt, host);
+}
+
+// Whether a list of n ids against a destination pool of `blocks` blocks (0: none) is
+// checked by the one workgroup of ids_check: its bitmap fits 32 KiB of LDS and each
+// thread holds its ids in registers. Beyond, the three launches over a bitmap in
+// memory spread the list over the device.
+bool one_launch_check(int32_t n, int64_t blocks) { return n <= kCheckIds && blocks <= kCheckBlocks; }
+
+int launch_check(const iekv_pool* src, const int32_t* src_ids, const iekv_pool* dst,
+                 const int32_t* dst_ids, int32_t n, bool same_pool, int32_t* checked,
+                 int32_t* status, hipStream_t stream) {
+  const int64_t blocks = dst ? dst->num_blocks : 0;
+  const uint32_t lds = static_cast<uint32_t>((blocks + 31) / 32 * sizeof(uint32_t));
+  hipLaunchKernelGGL(ids_check, dim3(1), dim3(kCheckThreads), lds, stream,
+                     src ? src_ids : nullptr, dst ? dst_ids : nullptr, n,
+                     src ? src->num_blocks : 0, blocks, same_pool ? 1 : 0, checked, status);
+  IEKV_HIP(hipGetLastError());
+  return IEKV_OK;
 }
 
 // One scatter of rows (iekv_write_slots_*): where they come from, where they go, and
@@ -3189,6 +3276,66 @@ int iekv_offload_blocks_ids(const iekv_pool* src, const int32_t* src_ids, int32_
                         compute, copy);
 }
 
+int iekv_copy_direct_checked(const iekv_pool* src, const iekv_pool* dst, const int32_t* src_ids,
+                             const int32_t* dst_ids, int32_t n_blocks, int32_t* checked,
+                             int32_t* status, hipStream_t stream, int32_t* bits) {
+  int rc;
+  if (!bits) return set_error(IEKV_ERR_INVALID, "bits is null");
+  if ((rc = check_pool(src, "source")) || (rc = check_pool(dst, "destination")) ||
+      (rc = check_ids(src_ids, n_blocks, "source")) ||
+      (rc = check_ids(dst_ids, n_blocks, "destination")))
+    return rc;
+  if (src->n_arrays != dst->n_arrays || src->tile_bytes != dst->tile_bytes)
+    return set_error(IEKV_ERR_INVALID, "pools differ in shape");
+  if (src->device != dst->device)
+    return set_error(IEKV_ERR_INVALID, "pools live on devices %d and %d", src->device,
+                     dst->device);
+  bool same_pool = false;
+  if ((rc = check_aliasing(src, dst, &same_pool))) return rc;
+  if (!one_launch_check(n_blocks, dst->num_blocks))
+    return set_error(IEKV_ERR_CAPACITY, "%d ids into %lld blocks: at most %d and %lld", n_blocks,
+                     static_cast<long long>(dst->num_blocks), kCheckIds,
+                     static_cast<long long>(kCheckBlocks));
+  *bits = 0;
+  if (n_blocks == 0) return IEKV_OK;
+  if (!checked || !status) return set_error(IEKV_ERR_INVALID, "checked or status is null");
+  if (reinterpret_cast<uintptr_t>(status) % alignof(int32_t) ||
+      reinterpret_cast<uintptr_t>(checked) % alignof(int32_t))
+    return set_error(IEKV_ERR_INVALID, "checked or status is not 4-byte aligned");
+  DeviceGuard guard(src->device);
+  if (!guard.ok()) return guard.fail();
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  IEKV_HIP(hipStreamIsCapturing(stream, &capture));
+  if (capture != hipStreamCaptureStatusNone)
+    return set_error(IEKV_ERR_INVALID, "a checked copy waits for its check: not under capture");
+  char* word = device_view_of_host(status, sizeof(int32_t));
+  if (!word) return set_error(IEKV_ERR_INVALID, "status is not pinned host memory");
+  constexpr int32_t kPending = -1;   // no set of IEKV_IDS_* bits
+  __atomic_store_n(status, kPending, __ATOMIC_RELEASE);
+  if ((rc = launch_check(src, src_ids, dst, dst_ids, n_blocks, same_pool, checked,
+                         reinterpret_cast<int32_t*>(word), stream)))
+    return rc;
+  rc = launch_move<true, true>(src, dst, nullptr, nullptr, checked, checked + n_blocks, n_blocks,
+                               src->tile_bytes, src->n_arrays, std::min(src->align, dst->align),
+                               stream);
+  // The word arrives while the move runs. Should the stream fail, or end without
+  // it, the query says so.
+  int32_t found;
+  for (uint32_t spin = 1; (found = __atomic_load_n(status, __ATOMIC_ACQUIRE)) == kPending; ++spin) {
+    if (spin % 16384 == 0) {
+      const hipError_t e = hipStreamQuery(stream);
+      if (e == hipErrorNotReady) continue;
+      (void)hipGetLastError();
+      if ((found = __atomic_load_n(status, __ATOMIC_ACQUIRE)) != kPending) break;
+      return set_error(IEKV_ERR_HIP, "the id check did not run: %s", hipGetErrorString(e));
+    }
+    __builtin_ia32_pause();
+  }
+  if (rc) return rc;
+  *bits = found;
+  return IEKV_OK;
+}
+
 int iekv_check_ids(const iekv_pool* src, const int32_t* src_ids, const iekv_pool* dst,
                    const int32_t* dst_ids, int32_t n_blocks, void* workspace,
                    int64_t workspace_bytes, int32_t* status, hipStream_t stream) {
@@ -3210,6 +3357,8 @@ int iekv_check_ids(const iekv_pool* src, const int32_t* src_ids, const iekv_pool
     return set_error(IEKV_ERR_INVALID, "workspace is not 4-byte aligned");
   DeviceGuard guard((src ? src : dst)->device);
   if (!guard.ok()) return guard.fail();
+  if (one_launch_check(n_blocks, dst ? dst->num_blocks : 0))
+    return launch_check(src, src_ids, dst, dst_ids, n_blocks, same_pool, nullptr, status, stream);
   auto* bitmap = static_cast<uint32_t*>(workspace);
   const uint32_t clear_grid =
       static_cast<uint32_t>(std::clamp<int64_t>((words + kThreads - 1) / kThreads, 1, 4096));

@@ -42,6 +42,10 @@ IEKV_IDS_DST_REPEATED = 4
 IEKV_IDS_OVERLAP = 8
 
 
+CHECK_ONE_LAUNCH_IDS = 8192          # IEKV_CHECK_ONE_LAUNCH_IDS
+CHECK_ONE_LAUNCH_BLOCKS = 262144     # IEKV_CHECK_ONE_LAUNCH_BLOCKS
+
+
 def check_workspace_bytes(num_blocks: int) -> int:
     """Workspace iekv_check_ids needs for a destination pool of num_blocks blocks."""
     return (num_blocks + 31) // 32 * 4
@@ -101,6 +105,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                 POINTER(c_int32), POINTER(c_int32), POINTER(c_int32)]),
     "iekv_check_ids": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_void_p,
                                c_int64, c_void_p, c_void_p]),
+    "iekv_copy_direct_checked": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int32,
+                                         c_void_p, c_void_p, c_void_p, POINTER(c_int32)]),
     "iekv_host_alloc": (c_int, [c_int64, POINTER(c_void_p)]),
     "iekv_host_free": (c_int, [c_void_p]),
     "iekv_noop": (c_int, [c_int32, c_int32, c_void_p]),

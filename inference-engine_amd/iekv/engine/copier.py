@@ -44,7 +44,7 @@ import torch
 
 from .. import _native
 from .pools import (KVPool, StreamScope, check_device_ids, current_stream_handle, host_buffer,
-                    integer_ids, stage_ids, stream_handle)
+                    integer_ids, raise_for_id_bits, stage_ids, stream_handle)
 
 # Device staging the host pipelines use: two slots of at most this many bytes.
 HOST_STAGING_BYTES = 256 << 20
@@ -846,6 +846,20 @@ class HipSlotCopier:
             if src.numel() != dst.numel():
                 raise ValueError(f"{src.numel()} source blocks for {dst.numel()} destinations")
             n = dst.numel()
+            if self.check_device_ids and n and n <= _native.CHECK_ONE_LAUNCH_IDS and \
+                    self.pool.num_blocks <= _native.CHECK_ONE_LAUNCH_BLOCKS:
+                with self._on(on):      # scratch of the stream the copy reads it on
+                    checked = torch.empty(2 * n, dtype=torch.int32, device=self.device)
+                word = torch.empty(1, dtype=torch.int32, pin_memory=True)
+                bits = ctypes.c_int32()
+                _native.call("iekv_copy_direct_checked", source.pool.native.handle,
+                             self.pool.native.handle, src.data_ptr(), dst.data_ptr(), n,
+                             checked.data_ptr(), word.data_ptr(), stream,
+                             ctypes.byref(bits))
+                raise_for_id_bits(bits.value, source.pool, self.pool)
+                source.blocks_read += n
+                self.blocks_written += n
+                return
             if self.check_device_ids:
                 with self._on(on):
                     check_device_ids(source.pool, src, self.pool, dst)

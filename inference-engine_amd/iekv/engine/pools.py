@@ -349,7 +349,11 @@ def check_device_ids(src_pool: KVPool | None, src_ids: torch.Tensor | None,
                  n, workspace.data_ptr() if dst_pool is not None else None,
                  workspace.numel() * 4 if dst_pool is not None else 0, status.data_ptr(),
                  current_stream_handle(owner.device))
-    bits = int(status.item())
+    raise_for_id_bits(int(status.item()), src_pool, dst_pool)
+
+
+def raise_for_id_bits(bits: int, src_pool: KVPool | None, dst_pool: KVPool | None) -> None:
+    """IndexError or ValueError for the IEKV_IDS_* bits of a failed check."""
     if bits & _native.IEKV_IDS_SRC_RANGE:
         raise IndexError(f"source block id out of range for a pool of "
                          f"{src_pool.num_blocks} blocks")

@@ -229,3 +229,58 @@ def test_the_checks_at_the_top_of_a_pool_of_int32_max_blocks(gpu):
     pool.native.close()
     del pool
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025, 8192, 8193])
+@pytest.mark.parametrize("blocks", [16500, 262144, 262145])
+def test_checked_copies_around_the_one_launch_limits(gpu, n, blocks):
+    """Lists and pools on either side of what one workgroup checks: a valid list moves its
+    blocks, one with a problem at any place raises and moves nothing, and the next valid
+    one is not held up by it. The bare check reports the same bits as NumPy's sets."""
+    from iekv.engine.copier import HipSlotCopier
+    from iekv.engine.pools import allocate_pool
+
+    def copier(seed):
+        k, v = allocate_pool(blocks, 1, 1, 1, 16, dtype=torch.uint8, device=gpu, zero=False)
+        k[0]._base.random_(0, 256, generator=torch.Generator(gpu).manual_seed(seed))
+        return HipSlotCopier(k, v, 1, check_device_ids=True)
+
+    src, dst = copier(1), copier(2)
+    rng = np.random.default_rng(n + blocks)
+    src_pool, dst_pool = src.pool, dst.pool
+    for plant in ("none", "src_low", "src_high", "dst_low", "dst_high", "repeat", "none"):
+        s = rng.integers(0, blocks, size=n)
+        d = rng.permutation(blocks)[:n]
+        at = int(rng.integers(n))
+        if plant == "src_low":
+            s[at] = -1
+        elif plant == "src_high":
+            s[at] = blocks
+        elif plant == "dst_low":
+            d[at] = -2**31
+        elif plant == "dst_high":
+            d[at] = blocks
+        elif plant == "repeat" and n > 1:
+            d[at] = d[at - 1]
+        bits = expected_bits(s, d, blocks, blocks, False)
+        assert run_check(src_pool, s, dst_pool, d) == bits
+        st, dt = (torch.from_numpy(x.astype(np.int32)).to(gpu) for x in (s, d))
+        want = [c.clone() for c in dst.k_caches + dst.v_caches]
+        if bits:
+            with pytest.raises((IndexError, ValueError)):
+                dst.copy_blocks(src, st, dt)
+        else:
+            dst.copy_blocks(src, st, dt)
+            for w, c in zip(want, src.k_caches + src.v_caches):
+                w[dt.long()] = c[st.long()]
+        torch.cuda.synchronize()
+        for w, c in zip(want, dst.k_caches + dst.v_caches):
+            assert torch.equal(w, c), plant
+    if 2 * n <= blocks and n > 1:
+        ids = rng.permutation(blocks)[:2 * n]
+        one = lambda x: torch.from_numpy(x.astype(np.int32)).to(gpu)
+        before = [c.clone() for c in dst.k_caches]
+        with pytest.raises(ValueError, match="disjoint"):
+            dst.copy_blocks(dst, one(ids[:n]), one(np.roll(ids[n - 1:2 * n - 1], 1)))
+        assert all(torch.equal(x, c) for x, c in zip(before, dst.k_caches))
+        dst.copy_blocks(dst, one(ids[:n]), one(ids[n:]))
