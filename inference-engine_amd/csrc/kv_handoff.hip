@@ -295,10 +295,8 @@ __device__ __forceinline__ void move_entry(const PoolView& src, const PoolView& 
 
 // Tiles smaller than a chunk: the workgroup moves tiles a0 .. a0 + group - 1
 // (arrays past n_arrays excepted) of list entry `entry`, i.e. one block's
-// tiles in `group` consecutive arrays. tile_vecs divides kThreads, so
-// lane t always takes vector t % tile_vecs of a tile: of tile
-// a0 + t / tile_vecs first, then of the tiles kThreads / tile_vecs further
-// on, with up to U of them in flight.
+// tiles in `group` consecutive arrays, laid end to end: lane t takes vectors
+// t, t + kThreads, ... of that run, with up to U of them in flight.
 template <typename V, int U, bool NT, bool SRC_POOL, bool DST_POOL>
 __device__ __forceinline__ void move_group(const PoolView& src, const PoolView& dst,
                                            const char* src_stage, char* dst_stage,
@@ -312,36 +310,40 @@ __device__ __forceinline__ void move_group(const PoolView& src, const PoolView& 
     if (dst_id < 0 || dst_id >= dst.num_blocks) return;
   }
   const int64_t tile_bytes = static_cast<int64_t>(tile_vecs) * sizeof(V);
-  const int t = threadIdx.x;
-  const int per_pass = kThreads / tile_vecs;
-  const int64_t lane_offset = static_cast<int64_t>(t % tile_vecs) * sizeof(V);
-  const int tiles = min(group, n_arrays - a0);
-  auto src_of = [&](int a) -> const char* {
-    if constexpr (SRC_POOL) return array_base(src, a) + src_id * tile_bytes + lane_offset;
-    else return src_stage + (entry * n_arrays + a) * tile_bytes + lane_offset;
+  const uint32_t vecs = static_cast<uint32_t>(min(group, n_arrays - a0)) * tile_vecs;
+  // The source and destination of vector e of the run; the division finds its tile.
+  auto place = [&](uint32_t e, gptr<const V>* s, gptr<V>* d) {
+    const uint32_t j = e / static_cast<uint32_t>(tile_vecs);
+    const int a = a0 + static_cast<int>(j);
+    const int64_t at = static_cast<int64_t>(e - j * tile_vecs) * sizeof(V);
+    if constexpr (SRC_POOL) *s = as_global<V>(array_base(src, a) + src_id * tile_bytes + at);
+    else *s = as_global<V>(src_stage + (entry * n_arrays + a) * tile_bytes + at);
+    if constexpr (DST_POOL) *d = as_global<V>(array_base(dst, a) + dst_id * tile_bytes + at);
+    else *d = as_global<V>(dst_stage + (entry * n_arrays + a) * tile_bytes + at);
   };
-  auto dst_of = [&](int a) -> char* {
-    if constexpr (DST_POOL) return array_base(dst, a) + dst_id * tile_bytes + lane_offset;
-    else return dst_stage + (entry * n_arrays + a) * tile_bytes + lane_offset;
-  };
-  for (int j = t / tile_vecs; j < tiles; j += U * per_pass) {
+  for (uint32_t e = threadIdx.x; e < vecs; e += U * kThreads) {
     V r[U];
+    gptr<V> to[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (e + u * kThreads < vecs) {
+        gptr<const V> from;
+        place(e + u * kThreads, &from, &to[u]);
+        r[u] = load_vec<V, NT>(from);
+      }
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (j + u * per_pass < tiles)
-        r[u] = load_vec<V, NT>(as_global<V>(src_of(a0 + j + u * per_pass)));
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (j + u * per_pass < tiles)
-        store_vec<V, NT>(as_global<V>(dst_of(a0 + j + u * per_pass)), r[u]);
+      if (e + u * kThreads < vecs) store_vec<V, NT>(to[u], r[u]);
   }
 }
 
 // One list entry's share of a workgroup: chunk p of its tile in array a, or,
 // with group > 1, its tiles in arrays a * group .. a * group + group - 1. The
-// grouped path keeps at most 4 vectors per lane in flight: each one carries
-// its own source and destination address, and at 8 the kernel's register
-// count would lower the occupancy of every launch it serves.
+// grouped path keeps at most 2 vectors per lane in flight: each one carries
+// its own source and destination address, and 4 were no faster (96-vector tiles
+// of 160 arrays 85.3 us against 85.2) while they took every launch that keeps 4
+// or more in flight from 62 to 76 VGPRs.
 template <typename V, int U, bool NT, bool SRC_POOL, bool DST_POOL, bool HOST = false>
 __device__ __forceinline__ void move_unit(const PoolView& src, const PoolView& dst,
                                           const char* src_stage, char* dst_stage,
@@ -349,7 +351,7 @@ __device__ __forceinline__ void move_unit(const PoolView& src, const PoolView& d
                                           int a, int p, int32_t tile_vecs, int32_t parts,
                                           int32_t group, int32_t n_arrays) {
   if (group > 1)
-    move_group<V, (U < 4 ? U : 4), NT, SRC_POOL, DST_POOL>(
+    move_group<V, (U < 2 ? U : 2), NT, SRC_POOL, DST_POOL>(
         src, dst, src_stage, dst_stage, src_id, dst_id, entry, a * group, tile_vecs, group,
         n_arrays);
   else
@@ -990,6 +992,7 @@ int plan_move(int32_t n_blocks, int64_t tile_bytes, int32_t n_arrays, int align,
     case iekv_plan::kTooManyArrays:
       return set_error(IEKV_ERR_INVALID, "%d arrays exceed the grid limit", n_arrays);
     default:
+      iekv_plan::group_ragged_tiles(tile_bytes, n_arrays, settings, pl);
       return IEKV_OK;
   }
 }

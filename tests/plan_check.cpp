@@ -595,6 +595,43 @@ void check_sort() {
       }
 }
 
+// Small tiles whose vectors do not divide the lanes: groups cover every array once, hold
+// no more than the kernel's passes, waste no more lanes than one tile per workgroup, and
+// their launches fit the dispatch limit; other plans are left as plan_move made them.
+void check_ragged_groups() {
+  for (int64_t tile_vecs : {1, 2, 3, 12, 48, 50, 96, 100, 128, 160, 192, 200, 240, 255, 256, 300})
+    for (int32_t n_arrays : {1, 2, 7, 14, 56, 160})
+      for (int32_t n_blocks : {1, 193, 9000000})
+        for (int64_t chunk : {0, 64, 4096, 8192, 65536})
+          for (int run : {0, 3}) {
+            Settings s;
+            s.chunk_bytes = chunk;
+            s.run = run;
+            MovePlan was, pl;
+            if (plan_move(n_blocks, tile_vecs * 16, n_arrays, 16, true, false, s, &was) != kPlanned)
+              continue;
+            pl = was;
+            group_ragged_tiles(tile_vecs * 16, n_arrays, s, &pl);
+            const bool ragged = run == 0 && tile_vecs * 16 < chunk && tile_vecs < kThreads &&
+                                kThreads % tile_vecs != 0;
+            if (!ragged) {
+              EXPECT(pl.group == was.group && pl.units == was.units &&
+                         pl.runs_per_launch == was.runs_per_launch && pl.lane_vecs == was.lane_vecs,
+                     "a plan that is not ragged is left alone");
+              continue;
+            }
+            EXPECT(pl.group >= 1 && pl.group <= n_arrays, "group of at least one array");
+            EXPECT(pl.group == 1 || pl.group * tile_vecs <= kRaggedVecs, "group within the passes");
+            EXPECT(pl.units * pl.group >= n_arrays && (pl.units - 1) * pl.group < n_arrays,
+                   "units cover every array once");
+            EXPECT(pl.runs_per_launch >= 1 && pl.runs_per_launch <= pl.total_runs &&
+                       pl.runs_per_launch * pl.units <= kMaxGrid,
+                   "one launch fits the dispatch limit");
+            const int64_t passes = (pl.group * tile_vecs + kThreads - 1) / kThreads;
+            EXPECT(pl.units * passes <= n_arrays, "no more passes than one tile per workgroup");
+          }
+}
+
 int main() {
   check_queue_claims();
   for (int grid = 1; grid <= 4096; ++grid) check_xcd_grouped(grid);
@@ -660,6 +697,7 @@ int main() {
   check_pieces_and_slots();
   check_launch_chunk();
   check_sort();
+  check_ragged_groups();
 
   if (failures) {
     std::printf("%d failures\n", failures);

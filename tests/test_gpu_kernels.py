@@ -290,6 +290,44 @@ def test_tiles_smaller_than_a_chunk_are_grouped_bit_exact(gpu, bs, heads, dim, d
     assert all(np.array_equal(a, b) for a, b in zip(source, host_bytes(sk) + host_bytes(sv)))
 
 
+@pytest.mark.parametrize("bs,heads,dim,dtype,layers", [
+    (8, 3, 32, torch.uint8, 28),       # 48 vectors, 56 arrays: four groups, the last shorter
+    (16, 1, 80, torch.bfloat16, 3),    # 160 vectors: groups of three of six arrays
+    (1, 1, 24, torch.float16, 40),     # 3 vectors, 80 arrays in one group
+    (15, 1, 68, torch.float32, 2),     # 255 vectors: two tiles fill two passes but two lanes
+    (8, 1, 36, torch.float16, 5),      # 36 vectors, one group of ten arrays
+    (3, 1, 10, torch.float16, 9),      # 15 vectors of 4 bytes
+])
+def test_ragged_small_tiles_are_grouped_bit_exact(gpu, bs, heads, dim, dtype, layers):
+    """Tiles of fewer than 256 vectors that do not divide a workgroup's lanes, at the default
+    launch shape: pack, unpack and direct copies with device ids and ids in the arguments,
+    an offload and a restore, against the oracle; the blocks beside stay as they are."""
+    from iekv.engine.copier import HipSlotCopier
+
+    sk, sv = allocate(60, bs, layers, heads, dim, dtype, gpu, seed=60)
+    dk, dv = allocate(50, bs, layers, heads, dim, dtype, gpu, seed=61)
+    src, dst = HipSlotCopier(sk, sv, bs), HipSlotCopier(dk, dv, bs)
+    rng = np.random.default_rng(62)
+    src_ids, dst_ids = random_tables(rng, 60, 50, 37)
+    src_o, dst_o = oracle_of(sk, sv, bs), oracle_of(dk, dv, bs)
+    want = packed_image(pack(src_o, src_ids))
+    handoff(src_o, dst_o, [src_ids], [dst_ids])
+    start = [t.clone() for t in dk + dv]
+    dev = lambda ids: torch.tensor(ids, dtype=torch.int32, device=gpu)  # noqa: E731
+    for ids_of in (dev, list):
+        for where in ("device", "host"):
+            for t, was in zip(dk + dv, start):
+                t.copy_(was)
+            packed = src.read_blocks(ids_of(src_ids), location=where)
+            if where == "host":
+                packed.synchronize()
+            assert np.array_equal(packed.data.cpu().numpy(), want), (ids_of, where)
+            dst.write_blocks(ids_of(dst_ids[:20]), packed[:20])
+            dst.copy_blocks(src, ids_of(src_ids[20:]), ids_of(dst_ids[20:]))
+            torch.cuda.synchronize()
+            assert_pool_equals(dk, dv, dst_o)
+
+
 @pytest.mark.parametrize("count", [1, 64, 66, 128, 130, 255, 256, 257, 600, 1300])
 def test_host_ids_in_the_kernel_arguments_and_beyond(gpu, count):
     """Host id lists ride in the launches' kernel arguments (iekv_*_ids), 256 per
