@@ -200,10 +200,47 @@ __device__ __forceinline__ void store_vec(gptr<V> p, V v) {
   else *p = v;
 }
 
+constexpr int kBufferWordFormat = 0x00020000;   // buffer resource word 3: 32-bit data format
+
+// Where a workgroup stores a run of n vectors that starts at `at`, wave-uniform. With
+// IMAGE the run is part of an image in HBM that a kernel soon behind reads again (a
+// packed payload, a gathered context): its 16-byte vectors are written through the L2
+// with the device-coherence bit instead of the non-temporal hint, which sends them to
+// HBM to be fetched from there. The Infinity Cache (256 MB) can then still hold a
+// smaller image when its reader comes or its buffer is written again, and the L2 has
+// nothing left to write back when the kernel ends. The stores go through a buffer
+// resource, the form in which the compiler lets the bit be chosen. Measured on MI355X,
+// non-temporal -> this: packs of 67 MB 25.9 -> 19.6 us, 126 MB 41.0 -> 38.5, 405 MB
+// and more level; a pack and its unpack 53.5 -> 41-47, 90 -> 76-84, 275 -> 235 us, of
+// 2.7 GB level; gathers of 126 MB 41.4 -> 32.7, 67 MB 25.4 -> 22.1, 1 GB level. With
+// the hint and the bit both nothing is gained. Ordinary stores packed 67 MB in 20.4 us
+// and 405 MB in 130 (126 with the hint). An unpack that writes its pool this way or
+// reads with ordinary loads loses part of it (405 MB pack and unpack 254 and 270 us).
+constexpr int kImageStorePolicy = 16;   // sc1: device-coherent
+
+template <typename V, bool NT, bool IMAGE>
+struct RunOut {
+  static constexpr bool kThrough = IMAGE && NT && sizeof(V) == 16;
+  gptr<V> d;
+  __amdgpu_buffer_rsrc_t run;
+  __device__ __forceinline__ RunOut(gptr<V> at, int n) : d(at) {
+    // A run is at most a tile: kMaxTileBytes fits the resource.
+    if constexpr (kThrough)
+      run = __builtin_amdgcn_make_buffer_rsrc((void*)at, 0, n * 16, kBufferWordFormat);
+  }
+  __device__ __forceinline__ void store(int i, V v) const {
+    if constexpr (kThrough)
+      __builtin_amdgcn_raw_buffer_store_b128(v, run, i * 16, 0, kImageStorePolicy);
+    else
+      store_vec<V, NT>(d + i, v);
+  }
+};
+
 // Move one tile of `n` vectors from s to d. Lane t handles vectors
 // t, t+256, ..., issuing U loads before the U stores that consume them.
-template <typename V, int U, bool NT>
+template <typename V, int U, bool NT, bool IMAGE = false>
 __device__ __forceinline__ void move_tile(gptr<const V> s, gptr<V> d, int n) {
+  const RunOut<V, NT, IMAGE> out(d, n);
   const int t = threadIdx.x;
   int v = t;
   const int full = n - (U - 1) * kThreads;  // v < full: all U vectors of the step are in range
@@ -212,7 +249,7 @@ __device__ __forceinline__ void move_tile(gptr<const V> s, gptr<V> d, int n) {
 #pragma unroll
     for (int u = 0; u < U; ++u) r[u] = load_vec<V, NT>(s + v + u * kThreads);
 #pragma unroll
-    for (int u = 0; u < U; ++u) store_vec<V, NT>(d + v + u * kThreads, r[u]);
+    for (int u = 0; u < U; ++u) out.store(v + u * kThreads, r[u]);
   }
   if (v < n) {
     V r[U];
@@ -221,7 +258,7 @@ __device__ __forceinline__ void move_tile(gptr<const V> s, gptr<V> d, int n) {
       if (v + u * kThreads < n) r[u] = load_vec<V, NT>(s + v + u * kThreads);
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (v + u * kThreads < n) store_vec<V, NT>(d + v + u * kThreads, r[u]);
+      if (v + u * kThreads < n) out.store(v + u * kThreads, r[u]);
   }
 }
 
@@ -289,15 +326,15 @@ __device__ __forceinline__ void move_entry(const PoolView& src, const PoolView& 
   } else {
     d = dst_stage + (entry * n_arrays + a) * tile_bytes;
   }
-  move_tile<V, U, NT>(as_global<V>(s + chunk_offset), as_global<V>(d + chunk_offset),
-                      chunk_vecs);
+  move_tile<V, U, NT, SRC_POOL && !DST_POOL && !HOST>(
+      as_global<V>(s + chunk_offset), as_global<V>(d + chunk_offset), chunk_vecs);
 }
 
 // Tiles smaller than a chunk: the workgroup moves tiles a0 .. a0 + group - 1
 // (arrays past n_arrays excepted) of list entry `entry`, i.e. one block's
 // tiles in `group` consecutive arrays, laid end to end: lane t takes vectors
 // t, t + kThreads, ... of that run, with up to U of them in flight.
-template <typename V, int U, bool NT, bool SRC_POOL, bool DST_POOL>
+template <typename V, int U, bool NT, bool SRC_POOL, bool DST_POOL, bool HOST>
 __device__ __forceinline__ void move_group(const PoolView& src, const PoolView& dst,
                                            const char* src_stage, char* dst_stage,
                                            int32_t src_id, int32_t dst_id, int64_t entry,
@@ -311,6 +348,9 @@ __device__ __forceinline__ void move_group(const PoolView& src, const PoolView& 
   }
   const int64_t tile_bytes = static_cast<int64_t>(tile_vecs) * sizeof(V);
   const uint32_t vecs = static_cast<uint32_t>(min(group, n_arrays - a0)) * tile_vecs;
+  // In a staging image the group's tiles are one run.
+  const RunOut<V, NT, !DST_POOL && !HOST> out(
+      as_global<V>(DST_POOL ? nullptr : dst_stage + (entry * n_arrays + a0) * tile_bytes), vecs);
   // The source and destination of vector e of the run; the division finds its tile.
   auto place = [&](uint32_t e, gptr<const V>* s, gptr<V>* d) {
     const uint32_t j = e / static_cast<uint32_t>(tile_vecs);
@@ -319,7 +359,6 @@ __device__ __forceinline__ void move_group(const PoolView& src, const PoolView& 
     if constexpr (SRC_POOL) *s = as_global<V>(array_base(src, a) + src_id * tile_bytes + at);
     else *s = as_global<V>(src_stage + (entry * n_arrays + a) * tile_bytes + at);
     if constexpr (DST_POOL) *d = as_global<V>(array_base(dst, a) + dst_id * tile_bytes + at);
-    else *d = as_global<V>(dst_stage + (entry * n_arrays + a) * tile_bytes + at);
   };
   for (uint32_t e = threadIdx.x; e < vecs; e += U * kThreads) {
     V r[U];
@@ -334,7 +373,10 @@ __device__ __forceinline__ void move_group(const PoolView& src, const PoolView& 
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      if (e + u * kThreads < vecs) store_vec<V, NT>(to[u], r[u]);
+      if (e + u * kThreads < vecs) {
+        if constexpr (DST_POOL) store_vec<V, NT>(to[u], r[u]);
+        else out.store(e + u * kThreads, r[u]);
+      }
   }
 }
 
@@ -351,7 +393,7 @@ __device__ __forceinline__ void move_unit(const PoolView& src, const PoolView& d
                                           int a, int p, int32_t tile_vecs, int32_t parts,
                                           int32_t group, int32_t n_arrays) {
   if (group > 1)
-    move_group<V, (U < 2 ? U : 2), NT, SRC_POOL, DST_POOL>(
+    move_group<V, (U < 2 ? U : 2), NT, SRC_POOL, DST_POOL, HOST>(
         src, dst, src_stage, dst_stage, src_id, dst_id, entry, a * group, tile_vecs, group,
         n_arrays);
   else
@@ -653,10 +695,11 @@ __device__ __forceinline__ void gather_share(const PoolView& pool, int32_t first
   const uint32_t block0 = base / sh.tile_vecs;
   const uint32_t offset0 = base - block0 * sh.tile_vecs;
   const char* src = array_base(pool, first_array + y);
-  const gptr<V> d = as_global<V>(out + y * out_stride) + base;
   const int64_t tile_bytes = static_cast<int64_t>(sh.tile_vecs) * sizeof(V);
   const uint32_t t = threadIdx.x;
   const uint32_t left = sh.vecs - base;   // > 0: the last workgroup may hold fewer
+  const RunOut<V, NT, true> d(as_global<V>(out + y * out_stride) + base,
+                                min(left, static_cast<uint32_t>(kThreads * U)));
   V v[U];
   bool have[U];
 #pragma unroll
@@ -677,7 +720,7 @@ __device__ __forceinline__ void gather_share(const PoolView& pool, int32_t first
   }
 #pragma unroll
   for (int u = 0; u < U; ++u)
-    if (have[u]) store_vec<V, NT>(d + u * kThreads + t, v[u]);
+    if (have[u]) d.store(u * kThreads + t, v[u]);
 }
 
 template <typename V, int U, bool NT, bool SPANS>
@@ -897,10 +940,10 @@ InlineKernel<W> pick_inline_kernel_as(int align, int unroll, int lane_vecs, bool
 #define IEKV_EXTRA
 #undef IEKV_PICK
 
-// The kernels of a move; `host`: an unpack that reads pinned host memory (move_entry's
-// HOST variant). Only unpacks have one.
+// The kernels of a move; `host`: an unpack that reads pinned host memory, or a pack that
+// writes it (the HOST variants of move_entry and move_group).
 #define IEKV_PICK_HOST(NAME)                                                                    \
-  if constexpr (!SP && DP) {                                                                    \
+  if constexpr (SP != DP) {                                                                     \
     if (host) return NAME##_as<SP, DP, true IEKV_EXTRA>(align, unroll, lane_vecs, nt, vec_bytes); \
   }                                                                                             \
   return NAME##_as<SP, DP, false IEKV_EXTRA>(align, unroll, lane_vecs, nt, vec_bytes);
@@ -1910,7 +1953,7 @@ int run_offload(const iekv_pool* src, IdList src_ids, int32_t n_blocks, void* ho
       char* piece = mapped + first * block_bytes;
       const int zc_align = std::min(src->align, align_of_ptr(reinterpret_cast<uint64_t>(piece)));
       const int rc = launch_list<true, false>(src, nullptr, piece, src_ids.from(first), cnt,
-                                              zc_align, compute, -1, nt);
+                                              zc_align, compute, -1, nt, true);
       if (rc) return rc;
     }
     return IEKV_OK;
@@ -2060,7 +2103,7 @@ int offload_images(const iekv_pool* src, IdList src_ids, int32_t n_blocks,
       std::copy(views.begin() + first, views.begin() + first + cnt, images.addr);
       const int32_t* device_ids = src_ids.on_host ? nullptr : src_ids.ids + first;
       if (src_ids.on_host) std::copy(src_ids.ids + first, src_ids.ids + first + cnt, images.ids);
-      if ((rc = launch_images<true, false>(src, images, device_ids, cnt, compute, -1, nt)))
+      if ((rc = launch_images<true, false>(src, images, device_ids, cnt, compute, -1, nt, true)))
         return rc;
     }
     return IEKV_OK;
@@ -2446,7 +2489,6 @@ __device__ void queue_leader(const QueueArgs& q, uint64_t start) {
 // less, a 16-byte vector as two.
 constexpr bool kQueueTileBufferStores = true;
 constexpr int kQueueStorePolicy = 16;        // sc1: device-coherent
-constexpr int kBufferWordFormat = 0x00020000;   // buffer resource word 3: 32-bit data format
 
 template <typename V>
 __device__ __forceinline__ void queue_store(gptr<V> p, V v) {

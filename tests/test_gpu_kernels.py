@@ -328,6 +328,50 @@ def test_ragged_small_tiles_are_grouped_bit_exact(gpu, bs, heads, dim, dtype, la
             assert_pool_equals(dk, dv, dst_o)
 
 
+@pytest.mark.parametrize("bs,heads,dim,dtype,context", [
+    (1, 1, 8, torch.float16, 5),          # 1 vector: groups of every array
+    (16, 5, 16, torch.float16, 33),       # 160 vectors: ragged groups
+    (257, 1, 8, torch.float16, 258),      # 257 vectors: a second pass of one lane
+    (16, 8, 128, torch.bfloat16, 47),     # 2,048 vectors: eight chunks of one pass
+    (25, 4, 128, torch.float32, 26),      # 3,200 vectors: chunks of a pass and a half
+    (3, 1, 10, torch.float16, 7),         # 4-byte vectors
+])
+def test_images_are_written_to_their_last_byte_and_no_further(gpu, bs, heads, dim, dtype, context):
+    """Packs and gathers into the middle of a larger buffer: the image is the oracle's, the
+    bytes around it stay, and an unpack right behind reads it."""
+    from iekv import _native
+    from iekv.engine.copier import HipSlotCopier
+    from iekv.engine.pools import current_stream_handle
+
+    layers = 3
+    sk, sv = allocate(40, bs, layers, heads, dim, dtype, gpu, seed=63)
+    dk, dv = allocate(40, bs, layers, heads, dim, dtype, gpu, seed=64)
+    src, dst = HipSlotCopier(sk, sv, bs), HipSlotCopier(dk, dv, bs)
+    src_ids, dst_ids = random_tables(np.random.default_rng(65), 40, 40, 17)
+    src_o, dst_o = oracle_of(sk, sv, bs), oracle_of(dk, dv, bs)
+    want = packed_image(pack(src_o, src_ids))
+    handoff(src_o, dst_o, [src_ids], [dst_ids])
+    payloads = src.empty_payloads(21)
+    payloads.data.fill_(0xA5)
+    dst.write_blocks(dst_ids, src.read_blocks(src_ids, into=payloads[2:19]))
+    got = payloads.data.cpu().numpy()
+    assert np.array_equal(got[2:19], want)
+    assert (got[:2] == 0xA5).all() and (got[19:] == 0xA5).all()
+    assert_pool_equals(dk, dv, dst_o)
+
+    table = torch.tensor(src_ids, dtype=torch.int32, device=gpu)
+    row = src.pool.tile_bytes // bs
+    size = 2 * layers * context * row
+    out = torch.full((size + 512,), 0xA5, dtype=torch.uint8, device=gpu)
+    _native.call("iekv_gather_rows_arrays", src.pool.native.handle, 0, 2 * layers, bs,
+                 table.data_ptr(), context, out.data_ptr() + 256, size,
+                 current_stream_handle(src.device))
+    got = out.cpu().numpy()
+    rows = want.transpose(1, 0, 2).reshape(2 * layers, -1)[:, :context * row]
+    assert np.array_equal(got[256:256 + size], rows.reshape(-1))
+    assert (got[:256] == 0xA5).all() and (got[256 + size:] == 0xA5).all()
+
+
 @pytest.mark.parametrize("count", [1, 64, 66, 128, 130, 255, 256, 257, 600, 1300])
 def test_host_ids_in_the_kernel_arguments_and_beyond(gpu, count):
     """Host id lists ride in the launches' kernel arguments (iekv_*_ids), 256 per
