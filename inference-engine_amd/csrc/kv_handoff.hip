@@ -1660,7 +1660,8 @@ int launch_write(const RowWrite& w, SlotList list, int32_t n_tokens, hipStream_t
 }
 
 // Vectors per lane of a gather workgroup: 4 KiB of 16-byte vectors per workgroup.
-// Measured on MI355X with 1, 2 and 4: 8B shape, 7,777 tokens 318 / 333 / 334 us
+// Measured on MI355X with non-temporal stores (before RunOut's) and 1, 2 and 4: 8B
+// shape, 7,777 tokens 318 / 333 / 334 us
 // (6.41 TB/s at 1; row by row it took 354); 70B share, 8,000 tokens 418 / 444 / 413;
 // 1,000 tokens 43.6 / 44.0 / 45.6; 800-byte rows, 3,000 tokens 43.7 / 45.3 / 48.9.
 // XCD-grouped positions cost 3-12% everywhere at 1, so the gather keeps the plain
