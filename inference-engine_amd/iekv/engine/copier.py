@@ -934,6 +934,7 @@ class HipSlotCopier:
                 raise ValueError(f"stream on {st.device}, pool on {self.device}")
         if done_events is not None and len(done_events) != len(tables):
             raise ValueError(f"{len(done_events)} events for {len(tables)} requests")
+        tables = list(tables)       # read more than once below: an iterator's items are kept
         self.flush()
         current = torch.cuda.current_stream(self.device)
         if done_events is None and len(streams) == 1:
