@@ -115,3 +115,74 @@ def test_tables_given_as_an_iterator_all_move(moved, sizes, n_streams, form):
     given = zip([t[0] for t in tables], [t[1] for t in tables])
     assert sorted(sum(moved(given, n_streams), [])) == want
     assert sorted(sum(moved((t for t in tables), n_streams), [])) == want
+
+
+@pytest.mark.parametrize("n_streams,events", [(0, False), (3, False), (0, True), (2, True)])
+@pytest.mark.parametrize("sizes", [[], [7], [0, 3], [800, 700, 900], [1, 0, 2100, 30, 4]], ids=str)
+def test_launches_hold_their_requests_by_destination_id(moved, sizes, n_streams, events):
+    """Uploaded ids: one launch per request with events, one per stream without, each
+    holding its own requests' pairs in ascending destination order."""
+    tables = requests(sizes, np.array) if sizes else []
+    evs = [SimpleNamespace(cuda_event=1) for _ in sizes] if events else None
+    got = moved(tables, n_streams, evs)
+    step = len(sizes) if events else max(n_streams, 1)
+    want = [sorted(pairs(tables[k::step]), key=lambda p: p[1])
+            for k in range(min(step, len(sizes)))]
+    assert [g for g in got if g] == [w for w in want if w]
+
+
+@pytest.mark.parametrize("sizes", [[1500, 1500], [2049], [1000, 1000, 1000]], ids=str)
+def test_ids_of_lists_over_the_merge_limit_are_not_read_twice(sizes):
+    """Whether lists are merged is decided by their lengths: no id is read for arrays that
+    are then thrown away."""
+    reads = []
+
+    class Id:
+        def __index__(self):
+            reads.append(1)
+            return 0
+
+    assert copier_module._merged_tables([([Id()] * n, [Id()] * n) for n in sizes]) is None
+    assert not reads
+
+
+@pytest.mark.parametrize("bad,error", [
+    (([1, 2], [3, 3]), ValueError), (([1, 2], [3, BLOCKS]), IndexError),
+    (([-1, 2], [3, 4]), IndexError), (([1, 2], [2**31, 4]), IndexError),
+    (([2**40, 2], [3, 4]), IndexError), (([1, 2], [-2**31, 4]), IndexError)], ids=str)
+def test_uploaded_ids_are_refused_before_anything_is_enqueued(moved, bad, error):
+    pool = Pool(num_blocks=BLOCKS, native=SimpleNamespace(handle=None))
+    for n_streams in (0, 2):
+        with pytest.raises(error):
+            moved(requests([4, 4], np.array) + [tuple(map(np.array, bad))], n_streams)
+    with pytest.raises(ValueError, match="disjoint"):
+        moved([(np.array([1]), np.array([2])), (np.array([2]), np.array([3]))], 2,
+              pools=(pool, pool))
+
+
+def test_ordering_long_requests_costs_no_more_than_an_argsort_of_each():
+    """Host time of the ids of 64 requests of 256 pairs, on one stream and on two: one
+    sort of keys per launch against an argsort per request and a sort for repeats (which
+    an earlier lexsort over all pairs exceeded by half)."""
+    import time
+
+    pool = Pool(num_blocks=BLOCKS)
+    tables = requests([256] * 64, np.array)
+
+    def each():
+        src, dst = [], []
+        for s, d in tables:
+            order = np.argsort(d, kind="stable")
+            src.append(s[order])
+            dst.append(d[order])
+        return pool.host_ids(np.concatenate(src)), pool.host_ids(np.concatenate(dst), unique=True)
+
+    def seconds(work):
+        start = time.perf_counter()
+        work()
+        return time.perf_counter() - start
+
+    for counts in ([64 * 256], [32 * 256] * 2):
+        order = lambda: copier_module._launch_order(pool, pool, tables, counts)  # noqa: E731
+        times = [(seconds(order), seconds(each)) for _ in range(9)]
+        assert min(t[0] for t in times) < min(t[1] for t in times)
