@@ -1562,36 +1562,33 @@ constexpr int kSmallSlots = 64;
 constexpr int kLongSlots = IEKV_INLINE_IDS;
 
 // Launches a checked scatter whose rows are `row_vecs` vectors of Op::Src, in as many
-// launches as the slots in the arguments (host slots) and 32-bit vector numbers need.
+// launches as the slots in the arguments (host slots), 32-bit vector numbers and the
+// dispatch limit need (iekv_plan::cut_rows).
 template <typename Op, int U>
 int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t row_vecs,
                     hipStream_t stream) {
   const int64_t per_group = kThreads * U;
   const int32_t layers = w.pool->n_arrays / 2;
-  // per_group more than the last vector stays below 2^31 too.
-  int64_t per_launch = std::max<int64_t>(1, (INT32_MAX - 2 * per_group) / row_vecs);
-  if (list.on_host) per_launch = std::min<int64_t>(per_launch, kLongSlots);
-  const int64_t most = std::min<int64_t>(n_tokens, per_launch) * row_vecs;
-  if ((most + per_group - 1) / per_group * 2 * w.n_layers > kMaxGrid)
-    return set_error(IEKV_ERR_INVALID, "%d tokens in %d layers exceed one launch", n_tokens,
-                     w.n_layers);
+  const iekv_plan::RowCut cut = iekv_plan::cut_rows(
+      row_vecs, w.n_layers, per_group, list.on_host ? kLongSlots : INT32_MAX, kMaxGrid / 2);
   DeviceGuard guard(w.pool->device);
   if (!guard.ok()) return guard.fail();
   const bool nt = g_nontemporal.load() != 0;
   const PoolView view = view_of(w.pool);
   const int64_t pool_rows = w.pool->num_blocks * w.block_size;
-  for (int64_t first = 0; first < n_tokens; first += per_launch) {
-    const int32_t n = static_cast<int32_t>(std::min<int64_t>(per_launch, n_tokens - first));
+  // One launch: rows first .. first + n - 1 of layers l0 .. l0 + n_layers - 1 of the call.
+  auto launch = [&](int64_t first, int32_t n, int32_t l0, int32_t n_layers) -> int {
     ScatterShape sh;
     sh.row_vecs = static_cast<int32_t>(row_vecs);
     sh.vecs = static_cast<int32_t>(n * row_vecs);
     sh.chunks = static_cast<int32_t>((sh.vecs + per_group - 1) / per_group);
     sh.xcd = (g_order.load() & iekv_plan::kXcdGrouped) != 0 ? 1 : 0;
-    sh.groups = sh.chunks * 2 * w.n_layers;
-    const int64_t skip = first * row_vecs * static_cast<int64_t>(sizeof(typename Op::Src));
+    sh.groups = sh.chunks * 2 * n_layers;
+    const int64_t skip = l0 * w.layer_stride +
+                         first * row_vecs * static_cast<int64_t>(sizeof(typename Op::Src));
     auto go = [&](auto kernel, const auto& slots) {
       return dispatch(kernel, dim3(static_cast<uint32_t>(sh.groups)), stream, view, layers,
-                      w.first_layer, w.n_layers, w.k + skip, w.v + skip, w.layer_stride, slots,
+                      w.first_layer + l0, n_layers, w.k + skip, w.v + skip, w.layer_stride, slots,
                       pool_rows, sh);
     };
     auto inlined = [&](auto words) {
@@ -1601,17 +1598,20 @@ int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t 
       return nt ? go(kv_scatter_inline<Op, U, true, W>, slots)
                 : go(kv_scatter_inline<Op, U, false, W>, slots);
     };
-    int rc;
     if (!list.on_host) {
       const DeviceSlots slots{list.slots + first};
-      rc = nt ? go(kv_scatter_rows<Op, U, true>, slots) : go(kv_scatter_rows<Op, U, false>, slots);
-    } else if (n <= kSmallSlots) {
-      rc = inlined(std::integral_constant<int, kSmallSlots>{});
-    } else {
-      rc = inlined(std::integral_constant<int, kLongSlots>{});
+      return nt ? go(kv_scatter_rows<Op, U, true>, slots)
+                : go(kv_scatter_rows<Op, U, false>, slots);
     }
-    if (rc) return rc;
-  }
+    return n <= kSmallSlots ? inlined(std::integral_constant<int, kSmallSlots>{})
+                            : inlined(std::integral_constant<int, kLongSlots>{});
+  };
+  for (int32_t l0 = 0; l0 < w.n_layers; l0 += cut.arrays)
+    for (int64_t first = 0; first < n_tokens; first += cut.units)
+      if (const int rc = launch(first,
+                                static_cast<int32_t>(std::min(cut.units, n_tokens - first)), l0,
+                                std::min(cut.arrays, w.n_layers - l0)))
+        return rc;
   return IEKV_OK;
 }
 
@@ -1730,8 +1730,8 @@ int launch_gather_as(const iekv_pool* pool, int32_t first_array, GatherShape sh,
 }
 
 // A checked gather of context_len >= 1 rows of n_arrays arrays, in launches of as
-// many blocks as the table in the arguments holds (host tables) and as 32-bit
-// vector numbers reach.
+// many blocks as the table in the arguments holds (host tables), 32-bit vector
+// numbers reach and the dispatch limit takes (iekv_plan::cut_rows).
 int launch_gather(const iekv_pool* pool, int32_t first_array, int32_t n_arrays,
                   int32_t block_size, IdList table, int32_t context_len, char* out,
                   hipStream_t stream) {
@@ -1743,18 +1743,13 @@ int launch_gather(const iekv_pool* pool, int32_t first_array, int32_t n_arrays,
   vec = std::min(vec, align_of_ptr(static_cast<uint64_t>(out_stride)));
   const int64_t tile_vecs = pool->tile_bytes / vec;
   const int64_t per_group = kThreads * (vec == 16 ? kGatherU : 4);
-  // per_group more than the last vector stays below 2^31 too.
-  int64_t blocks_per_launch = std::max<int64_t>(1, (INT32_MAX - 2 * per_group) / tile_vecs);
-  if (table.on_host) blocks_per_launch = std::min<int64_t>(blocks_per_launch, kLongTable);
+  const iekv_plan::RowCut cut = iekv_plan::cut_rows(
+      tile_vecs, n_arrays, per_group, table.on_host ? kLongTable : INT32_MAX, kMaxGrid);
   const int64_t blocks = (static_cast<int64_t>(context_len) - 1) / block_size + 1;
-  const int64_t most = std::min(blocks, blocks_per_launch) * tile_vecs;
-  if ((most + per_group - 1) / per_group * n_arrays > kMaxGrid)
-    return set_error(IEKV_ERR_INVALID, "a context of %d rows in %d arrays exceeds one launch",
-                     context_len, n_arrays);
   DeviceGuard guard(pool->device);
   if (!guard.ok()) return guard.fail();
-  for (int64_t first = 0; first < blocks; first += blocks_per_launch) {
-    const int64_t count = std::min(blocks_per_launch, blocks - first);
+  // One launch: blocks first .. first + count - 1 of arrays a0 .. a0 + arrays - 1 of the call.
+  auto launch = [&](int64_t first, int32_t count, int32_t a0, int32_t arrays) -> int {
     const int64_t begin = first * pool->tile_bytes;
     const int64_t end = std::min((first + count) * pool->tile_bytes, out_stride);
     GatherShape sh;
@@ -1762,33 +1757,24 @@ int launch_gather(const iekv_pool* pool, int32_t first_array, int32_t n_arrays,
     sh.vecs = static_cast<int32_t>((end - begin) / vec);
     sh.chunks = static_cast<int32_t>((sh.vecs + per_group - 1) / per_group);
     sh.xcd = (g_pack_order.load() & iekv_plan::kXcdGrouped) != 0 ? 1 : 0;
-    sh.groups = sh.chunks * n_arrays;
-    const IdList part = table.from(first);
-    const int32_t n = static_cast<int32_t>(count);
-    int rc;
+    sh.groups = sh.chunks * arrays;
+    char* to = out + a0 * out_stride + begin;
+    auto go = [&](auto kernel) {
+      return kernel(pool, first_array + a0, sh, table.from(first), count, to, out_stride, stream);
+    };
     switch (vec) {
-      case 16:
-        rc = launch_gather_as<u32x4, kGatherU>(pool, first_array, sh, part, n, out + begin,
-                                               out_stride, stream);
-        break;
-      case 8:
-        rc = launch_gather_as<u32x2, 4>(pool, first_array, sh, part, n, out + begin, out_stride,
-                                        stream);
-        break;
-      case 4:
-        rc = launch_gather_as<uint32_t, 4>(pool, first_array, sh, part, n, out + begin,
-                                           out_stride, stream);
-        break;
-      case 2:
-        rc = launch_gather_as<uint16_t, 4>(pool, first_array, sh, part, n, out + begin,
-                                           out_stride, stream);
-        break;
-      default:
-        rc = launch_gather_as<uint8_t, 4>(pool, first_array, sh, part, n, out + begin,
-                                          out_stride, stream);
+      case 16: return go(launch_gather_as<u32x4, kGatherU>);
+      case 8: return go(launch_gather_as<u32x2, 4>);
+      case 4: return go(launch_gather_as<uint32_t, 4>);
+      case 2: return go(launch_gather_as<uint16_t, 4>);
+      default: return go(launch_gather_as<uint8_t, 4>);
     }
-    if (rc) return rc;
-  }
+  };
+  for (int32_t a0 = 0; a0 < n_arrays; a0 += cut.arrays)
+    for (int64_t first = 0; first < blocks; first += cut.units)
+      if (const int rc = launch(first, static_cast<int32_t>(std::min(cut.units, blocks - first)),
+                                a0, std::min(cut.arrays, n_arrays - a0)))
+        return rc;
   return IEKV_OK;
 }
 

@@ -237,6 +237,28 @@ inline void group_ragged_tiles(int64_t tile_bytes, int32_t n_arrays, const Setti
   pl->runs_per_launch = pl->total_runs < fit ? pl->total_runs : fit;
 }
 
+// One launch of a row kernel (a scatter, whose units are rows, or a gather, whose units are
+// blocks): `units` units of unit_vecs vectors in each of `arrays` arrays, per_group vectors
+// to a workgroup that works in one array. A launch holds at most most_groups workgroups, a
+// vector's number in its array stays per_group below 2^31 for the lanes past the last one,
+// and at most most_units units (ids that ride in the arguments). Larger calls take several
+// launches, which also cut the arrays where one unit of all of them is too much.
+struct RowCut {
+  int64_t units;
+  int32_t arrays;
+};
+
+inline RowCut cut_rows(int64_t unit_vecs, int32_t n_arrays, int64_t per_group,
+                       int64_t most_units, int64_t most_groups) {
+  RowCut cut;
+  const int64_t unit_groups = (unit_vecs + per_group - 1) / per_group;
+  cut.arrays = static_cast<int32_t>(std::clamp<int64_t>(most_groups / unit_groups, 1, n_arrays));
+  const int64_t most_vecs = std::min(INT32_MAX - 2 * per_group,
+                                     most_groups / cut.arrays * per_group);
+  cut.units = std::clamp<int64_t>(most_vecs / unit_vecs, 1, most_units);
+  return cut;
+}
+
 // Workgroups of one launch of a plan that covers `runs` runs (at most
 // runs_per_launch): every launch of the move kernels has exactly this many,
 // and the kernels rely on it (place_in_grid derives the grid size from the

@@ -632,7 +632,44 @@ void check_ragged_groups() {
           }
 }
 
+// Cuts of the row kernels' calls: every launch within the dispatch limit, 32-bit vector
+// numbers and the ids its arguments hold; the launches cover every (array, unit) once; and
+// no launch is cut further than one of the limits asks.
+void check_row_cuts() {
+  for (int64_t unit_vecs : {1ll, 3ll, 64ll, 128ll, 2048ll, 65537ll, 1ll << 26, 1ll << 30})
+    for (int32_t n_arrays : {1, 2, 32, 64, 160, 70000})
+      for (int64_t per_group : {256, 512, 1024})
+        for (int64_t most_units : {int64_t(256), int64_t(512), int64_t(INT32_MAX)})
+          for (int64_t most_groups : {kMaxGrid, kMaxGrid / 2}) {
+            const RowCut c = cut_rows(unit_vecs, n_arrays, per_group, most_units, most_groups);
+            const auto groups = [&](int64_t units, int64_t arrays) {
+              return (units * unit_vecs + per_group - 1) / per_group * arrays;
+            };
+            EXPECT(c.units >= 1 && c.units <= most_units && c.arrays >= 1 && c.arrays <= n_arrays,
+                   "%lld units of %d arrays", (long long)c.units, c.arrays);
+            EXPECT(groups(c.units, c.arrays) <= most_groups, "%lld workgroups of at most %lld",
+                   (long long)groups(c.units, c.arrays), (long long)most_groups);
+            EXPECT(c.units * unit_vecs + 2 * per_group <= INT32_MAX, "%lld vectors of an array",
+                   (long long)(c.units * unit_vecs));
+            EXPECT(c.arrays == n_arrays || groups(1, c.arrays + 1) > most_groups,
+                   "arrays cut at %d of %d though one unit of more fits", c.arrays, n_arrays);
+            EXPECT(c.units == most_units ||
+                       (c.units + 1) * unit_vecs + 2 * per_group > INT32_MAX ||
+                       (c.units + 1) * unit_vecs > most_groups / c.arrays * per_group,
+                   "%lld units though more fit", (long long)c.units);
+          }
+  // The 8B shape's 524,287 and 1,048,572 tokens (2 KiB rows of 64 arrays): 64 and 128 GiB.
+  for (int64_t tokens : {524287ll, 1048572ll, 2147483647ll}) {
+    const RowCut c = cut_rows(128, 32, 256, INT32_MAX, kMaxGrid / 2);
+    EXPECT(c.arrays == 32 && (tokens + c.units - 1) / c.units <= 8192, "scatter launches");
+    const RowCut g = cut_rows(2048, 64, 256, INT32_MAX, kMaxGrid);
+    EXPECT(g.arrays == 64 && g.units * 16 >= 524272, "gather launches of %lld blocks",
+           (long long)g.units);
+  }
+}
+
 int main() {
+  check_row_cuts();
   check_queue_claims();
   for (int grid = 1; grid <= 4096; ++grid) check_xcd_grouped(grid);
   for (int grid : {98816, 1048575, 4194304, 16777215}) check_xcd_grouped(grid);

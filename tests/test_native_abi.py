@@ -630,3 +630,34 @@ def test_request_queue_arguments_are_checked_before_any_hip_call(lib):
     refused(lib.iekv_queue_stop(None), "queue is null")
     refused(lib.iekv_queue_stats(None, None, None), "queue is null")
     assert lib.iekv_queue_destroy(None) == _native.IEKV_OK
+
+
+@pytest.mark.parametrize("tokens", [524_272, 524_288, 1_048_572, 2**31 - 1])
+def test_row_calls_of_any_size_are_cut_into_launches_not_refused(lib, tokens):
+    """Writes by device slot and gathers through a device table over 64 arrays of 2 KiB rows,
+    with more 4 KiB workgroups than one dispatch holds: the call goes on to its device
+    (which does not exist, so nothing is launched) instead of refusing its size. So do
+    rows of 1 GiB, of which not even one of every array fits a dispatch."""
+    from iekv import _native
+
+    def reaches_its_device(rc):
+        assert rc == _native.IEKV_ERR_HIP, lib.iekv_last_error().decode()
+
+    row, rows = 2048, 2 ** 20
+    pool = _native.Pool([(1 << 44) + a * rows * row for a in range(64)], tile_bytes=16 * row,
+                        num_blocks=rows // 16, device=99)
+    at = 1 << 40        # never touched: an aligned address stands for the device buffers
+    stride = tokens * row
+    reaches_its_device(lib.iekv_write_slots_layers(pool.handle, 0, 32, 16, at, at, stride, at,
+                                                   tokens, None))
+    reaches_its_device(lib.iekv_gather_rows_arrays(pool.handle, 0, 64, 16, at, tokens, at,
+                                                   64 * stride, None))
+    pool.close()
+    big = _native.Pool([(1 << 44) + a * (1 << 31) for a in range(200)], tile_bytes=1 << 30,
+                       num_blocks=2, device=99)
+    for odd in (0, 1):  # 16-byte vectors, and single bytes
+        reaches_its_device(lib.iekv_write_slots_layers(big.handle, 0, 100, 1, at + odd, at, 0, at,
+                                                       2, None))
+        reaches_its_device(lib.iekv_gather_rows_arrays(big.handle, 0, 200, 1, at, 2, at + odd,
+                                                       200 << 31, None))
+    big.close()
