@@ -57,6 +57,12 @@ def _slots(pool: KVPool, slots):
     if checked.min() < 0 or checked.max() >= rows:
         bad = checked[(checked < 0) | (checked >= rows)][0]
         raise IndexError(f"slot {bad} out of range for a pool of {rows} slots")
+    with torch.cuda.device(pool.device):
+        if torch.cuda.is_current_stream_capturing():
+            # A replay would read the pinned copy of the list again, long after it was freed.
+            raise RuntimeError(f"a list of {len(host)} slots is uploaded, which a stream under "
+                               f"capture cannot do: pass a device tensor, or at most "
+                               f"{HOST_SLOTS_MAX} slots")
     t = torch.from_numpy(checked).pin_memory().to(pool.device, non_blocking=True)
     return t, "iekv_write_slots_cast"
 

@@ -331,3 +331,35 @@ def test_rows_of_another_type_are_written_as_their_casts(gpu, bs, heads, dim, ro
         for bad in (-1, rows_in_pool):
             with pytest.raises(IndexError, match=f"slot {bad} out of range"):
                 write_slots_layers(pool, rows[0], rows[1], slots[:-1] + [bad])
+
+
+def test_captured_writes_replay_and_uploads_are_refused_under_capture(gpu):
+    """A list that rides in the launches' arguments and a device tensor are captured and
+    write the rows' present values on every replay; a longer list, which is uploaded from
+    memory that does not outlive the call, is refused and leaves the capture whole."""
+    from iekv.engine.slots import HOST_SLOTS_MAX, write_slots
+
+    k, v, pool = random_pool(70, 16, 2, 32, torch.float16, gpu, layers=1, seed=5)
+    n = HOST_SLOTS_MAX
+    order = np.random.default_rng(6).permutation(70 * 16)
+    slots, tensor = order[:n].tolist(), torch.from_numpy(order[n:2 * n].copy()).to(gpu)
+    rows = torch.zeros((n + 1, 2, 32), dtype=torch.float32, device=gpu)
+    write_slots(pool, 0, rows[:n], rows[:n], slots)      # first use outside the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        with pytest.raises(RuntimeError, match="under capture"):
+            write_slots(pool, 0, rows, rows, order[:n + 1].tolist())
+        write_slots(pool, 0, rows[:n], rows[:n], slots)
+        write_slots(pool, 0, rows[:n], rows[:n], tensor)
+    for step in range(4):
+        rows.copy_(torch.randn(rows.shape, device=gpu,
+                               generator=torch.Generator(gpu).manual_seed(step)))
+        want = [c.clone() for c in k + v]
+        for w in want:
+            w[torch.tensor(slots, device=gpu)] = rows[:n].half()
+            w[tensor] = rows[:n].half()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(w.view(torch.int16), c.view(torch.int16))
+                   for w, c in zip(want, k + v)), step      # bytes: the pool holds NaNs
