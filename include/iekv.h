@@ -54,7 +54,7 @@
 extern "C" {
 #endif
 
-#define IEKV_ABI_VERSION 21
+#define IEKV_ABI_VERSION 22
 
 enum {
   IEKV_OK = 0,

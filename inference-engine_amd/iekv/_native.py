@@ -12,7 +12,7 @@ from ctypes import POINTER, c_char_p, c_int, c_int32, c_int64, c_uint64, c_void_
 from pathlib import Path
 
 LIBRARY = Path(__file__).resolve().parent / "libiekv.so"
-ABI_VERSION = 21
+ABI_VERSION = 22
 
 INLINE_IDS = 256   # IEKV_INLINE_IDS: most host ids one launch carries in its arguments
 HOST_DIRECT_MAX = 64 << 20   # IEKV_HOST_DIRECT_MAX_BYTES: largest direct offload; restore launch size
@@ -170,13 +170,16 @@ def lib() -> ctypes.CDLL:
             f"{path} is missing: build it with `python -m iekv.build` or "
             "`python -c 'import __graft_entry__ as g; g.build()'` before using the HIP path")
     handle = ctypes.CDLL(str(path))
+    # The version first: a library of another one may lack entry points bound below.
+    handle.iekv_abi_version.restype, handle.iekv_abi_version.argtypes = \
+        SIGNATURES["iekv_abi_version"]
+    version = handle.iekv_abi_version()
+    if version != ABI_VERSION:
+        raise RuntimeError(f"{path} has ABI version {version}, expected {ABI_VERSION}")
     for name, (restype, argtypes) in SIGNATURES.items():
         fn = getattr(handle, name)
         fn.restype = restype
         fn.argtypes = argtypes
-    version = handle.iekv_abi_version()
-    if version != ABI_VERSION:
-        raise RuntimeError(f"{path} has ABI version {version}, expected {ABI_VERSION}")
     _lib = handle
     return handle
 

@@ -40,7 +40,7 @@ def test_every_declared_function_is_exported_and_bound(lib):
 
 
 def test_abi_version(lib):
-    assert lib.iekv_abi_version() == 21
+    assert lib.iekv_abi_version() == 22
 
 
 def test_pool_create_rejects_bad_arguments_before_touching_the_gpu(lib):
@@ -661,3 +661,30 @@ def test_row_calls_of_any_size_are_cut_into_launches_not_refused(lib, tokens):
         reaches_its_device(lib.iekv_gather_rows_arrays(big.handle, 0, 200, 1, at, 2, at + odd,
                                                        200 << 31, None))
     big.close()
+
+
+def test_a_library_of_an_older_interface_is_refused_by_its_version(tmp_path):
+    """A library that lacks entry points added since is refused by its ABI version, the
+    same as one that has them all, instead of by the first missing symbol."""
+    import os
+    import shutil
+    import subprocess
+    import sys
+
+    from iekv import _native
+
+    gcc = shutil.which("gcc")
+    if gcc is None:
+        pytest.skip("gcc is not installed")
+    stub = tmp_path / "older.c"
+    stub.write_text("int iekv_abi_version(void) { return 21; }\n")
+    library = tmp_path / "libiekv_older.so"
+    subprocess.run([gcc, "-shared", "-fPIC", str(stub), "-o", str(library)], check=True,
+                   capture_output=True, timeout=120)
+    probe = (f"import sys\nsys.path.insert(0, {str(ROOT / 'inference-engine_amd')!r})\n"
+             "from iekv import _native\n"
+             "try:\n    _native.lib()\nexcept RuntimeError as e:\n    print('refused:', e)\n")
+    out = subprocess.run([sys.executable, "-c", probe], capture_output=True, text=True,
+                         timeout=300, env=dict(os.environ, IEKV_LIBRARY=str(library)))
+    assert out.returncode == 0, out.stderr[-2000:]
+    assert f"ABI version 21, expected {_native.ABI_VERSION}" in out.stdout
