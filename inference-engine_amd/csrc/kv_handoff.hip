@@ -1018,10 +1018,11 @@ int32_t chunk_of(bool pool_reading, bool pool_writing, int64_t tile_bytes) {
 
 // The launch shape of one move under the current settings (kv_plan.h), with
 // chunk_of's chunk size; `chunk` >= 0 sets this launch's chunk size instead
-// (host_read_chunk for moves that read pinned host memory).
+// (host_read_chunk for moves that read pinned host memory); `host`: the launch reads or
+// writes pinned host memory.
 int plan_move(int32_t n_blocks, int64_t tile_bytes, int32_t n_arrays, int align,
               bool pool_reading, bool pool_writing, bool single_blocks, MovePlan* pl,
-              int32_t chunk = -1) {
+              int32_t chunk = -1, bool host = false) {
   iekv_plan::Settings settings;
   settings.run = g_run.load();
   settings.chunk_bytes = chunk >= 0 ? chunk : chunk_of(pool_reading, pool_writing, tile_bytes);
@@ -1035,7 +1036,8 @@ int plan_move(int32_t n_blocks, int64_t tile_bytes, int32_t n_arrays, int align,
     case iekv_plan::kTooManyArrays:
       return set_error(IEKV_ERR_INVALID, "%d arrays exceed the grid limit", n_arrays);
     default:
-      iekv_plan::group_ragged_tiles(tile_bytes, n_arrays, settings, pl);
+      iekv_plan::group_ragged_tiles(tile_bytes, n_arrays, settings,
+                                    iekv_plan::ragged_most_vecs(host, pool_writing), pl);
       return IEKV_OK;
   }
 }
@@ -1064,7 +1066,8 @@ int launch_move(const iekv_pool* sp, const iekv_pool* dp, const char* src_stage,
   if (n_blocks == 0) return IEKV_OK;
   MovePlan pl;
   int rc;
-  if ((rc = plan_move(n_blocks, tile_bytes, n_arrays, align, SP, DP, false, &pl, chunk)))
+  if ((rc = plan_move(n_blocks, tile_bytes, n_arrays, align, SP, DP, false, &pl, chunk,
+                      host)))
     return rc;
   MoveKernel k = pick_kernel<SP, DP>(align, g_unroll.load(), pl.lane_vecs, nontemporal(nt),
                                      &pl.vec, host);
@@ -1096,7 +1099,7 @@ int launch_move_inline(const iekv_pool* sp, const iekv_pool* dp, const char* src
   if (n_blocks == 0) return IEKV_OK;
   MovePlan pl;
   int rc;
-  if ((rc = plan_move(n_blocks, tile_bytes, n_arrays, align, SP, DP, true, &pl, chunk)))
+  if ((rc = plan_move(n_blocks, tile_bytes, n_arrays, align, SP, DP, true, &pl, chunk, host)))
     return rc;
   InlineKernel<W> k = pick_inline_kernel<SP, DP, W>(align, g_unroll.load(), pl.lane_vecs,
                                                     nontemporal(nt), &pl.vec, host);
@@ -1123,7 +1126,7 @@ int launch_images(const iekv_pool* pool, const InlineImages& images, const int32
   MovePlan pl;
   int rc;
   if ((rc = plan_move(n_blocks, pool->tile_bytes, pool->n_arrays, align, SP, DP, true, &pl,
-                      chunk)))
+                      chunk, host)))
     return rc;
   // At most IEKV_HOST_DIRECT_MAX_BYTES in chunks of at least 64 bytes: one launch holds them.
   if (pl.runs_per_launch < n_blocks)

@@ -220,12 +220,27 @@ inline int ragged_group(int64_t tile_vecs, int32_t n_arrays) {
   return 1;
 }
 
+// Largest tile, in vectors, that a launch groups so. Launches that go through pinned host
+// memory are bound by the host link, not by idle lanes: only the smallest tiles gain, and
+// from the limits below on fewer, larger workgroups keep the link less busy. Measured on
+// MI355X, one tile per workgroup against groups, 56 and 160 arrays, us: reads of 5-vector
+// tiles 129 -> 89 and 527 -> 318, 12 94 -> 94 and 363 -> 327, 17 86 -> 91 and 328 -> 321,
+// 24 78 -> 95 and 304 -> 327, 48 77 -> 97 and 296 -> 332, 96 87 -> 79 and 311 -> 347;
+// writes of 5 110 -> 82 and 454 -> 327, 24 81 -> 80 and 334 -> 338, 40 81 -> 80 and
+// 334 -> 331, 48 79 -> 79 and 326 -> 333, 96 78 -> 77 and 330 -> 335.
+constexpr int kRaggedHostReadVecs = 12;
+constexpr int kRaggedHostWriteVecs = 40;
+
+inline int ragged_most_vecs(bool host, bool pool_writing) {
+  return !host ? kThreads - 1 : pool_writing ? kRaggedHostReadVecs : kRaggedHostWriteVecs;
+}
+
 // Groups the tiles of a plan that plan_move left one per workgroup although they are
-// smaller than the chunk.
+// smaller than the chunk, up to tiles of most_vecs vectors.
 inline void group_ragged_tiles(int64_t tile_bytes, int32_t n_arrays, const Settings& s,
-                               MovePlan* pl) {
+                               int most_vecs, MovePlan* pl) {
   if (pl->run != 1 || pl->parts != 1 || pl->group != 1 || s.chunk_bytes <= 0 ||
-      tile_bytes >= s.chunk_bytes || pl->tile_vecs >= kThreads ||
+      tile_bytes >= s.chunk_bytes || pl->tile_vecs > most_vecs ||
       kThreads % pl->tile_vecs == 0)
     return;
   pl->group = ragged_group(pl->tile_vecs, n_arrays);

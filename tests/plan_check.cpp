@@ -603,7 +603,8 @@ void check_ragged_groups() {
     for (int32_t n_arrays : {1, 2, 7, 14, 56, 160})
       for (int32_t n_blocks : {1, 193, 9000000})
         for (int64_t chunk : {0, 64, 4096, 8192, 65536})
-          for (int run : {0, 3}) {
+          for (int which = 0; which < 6; ++which) {
+            const int run = which % 2 ? 3 : 0, most_vecs = which < 2 ? 255 : which < 4 ? 40 : 12;
             Settings s;
             s.chunk_bytes = chunk;
             s.run = run;
@@ -611,8 +612,8 @@ void check_ragged_groups() {
             if (plan_move(n_blocks, tile_vecs * 16, n_arrays, 16, true, false, s, &was) != kPlanned)
               continue;
             pl = was;
-            group_ragged_tiles(tile_vecs * 16, n_arrays, s, &pl);
-            const bool ragged = run == 0 && tile_vecs * 16 < chunk && tile_vecs < kThreads &&
+            group_ragged_tiles(tile_vecs * 16, n_arrays, s, most_vecs, &pl);
+            const bool ragged = run == 0 && tile_vecs * 16 < chunk && tile_vecs <= most_vecs &&
                                 kThreads % tile_vecs != 0;
             if (!ragged) {
               EXPECT(pl.group == was.group && pl.units == was.units &&
@@ -630,6 +631,10 @@ void check_ragged_groups() {
             const int64_t passes = (pl.group * tile_vecs + kThreads - 1) / kThreads;
             EXPECT(pl.units * passes <= n_arrays, "no more passes than one tile per workgroup");
           }
+  EXPECT(ragged_most_vecs(false, true) == kThreads - 1 && ragged_most_vecs(false, false) == 255,
+         "every small tile through HBM");
+  EXPECT(ragged_most_vecs(true, true) == 12 && ragged_most_vecs(true, false) == 40,
+         "only the smallest through the host link");
 }
 
 // Cuts of the row kernels' calls: every launch within the dispatch limit, 32-bit vector
