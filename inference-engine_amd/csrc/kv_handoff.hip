@@ -200,6 +200,25 @@ __device__ __forceinline__ void store_vec(gptr<V> p, V v) {
   else *p = v;
 }
 
+// The same at any address: a vector's bytes need not lie on its own multiple (one global
+// access still, at whatever width). The aligned forms above stay where alignment is known:
+// an access that straddles a cache line is two for the memory.
+template <typename V, bool NT>
+__device__ __forceinline__ V load_loose(const char* p) {
+  typedef const V L __attribute__((aligned(1)));
+  const auto q = (__attribute__((address_space(1))) L*)p;
+  if constexpr (NT) return __builtin_nontemporal_load(q);
+  else return *q;
+}
+
+template <typename V, bool NT>
+__device__ __forceinline__ void store_loose(char* p, V v) {
+  typedef V L __attribute__((aligned(1)));
+  const auto q = (__attribute__((address_space(1))) L*)p;
+  if constexpr (NT) __builtin_nontemporal_store(v, q);
+  else *q = v;
+}
+
 constexpr int kBufferWordFormat = 0x00020000;   // buffer resource word 3: 32-bit data format
 
 // Where a workgroup stores a run of n vectors that starts at `at`, wave-uniform. With
@@ -506,6 +525,7 @@ constexpr int kWave = 64;
 // with the slot read first).
 struct ScatterShape {
   int32_t row_vecs;   // source vectors per row
+  int32_t back;       // elements a row's last vector starts before the end of the one before it
   int32_t vecs;       // source vectors per layer in this launch (host: fits int32)
   int32_t chunks;     // workgroups per array
   int32_t xcd;        // 1: XCD-grouped workgroup positions
@@ -533,6 +553,7 @@ template <typename V>
 struct Bytes {
   using Src = V;
   using Dst = V;
+  static constexpr int kElems = sizeof(V), kSrcElem = 1, kDstElem = 1;   // bytes are the elements
   static __device__ __forceinline__ V run(V v) { return v; }
 };
 
@@ -585,6 +606,8 @@ template <typename From, typename To, int N>
 struct Cast {
   using Src = raw_bytes<N * sizeof(typename From::Elem)>;
   using Dst = raw_bytes<N * sizeof(typename To::Elem)>;
+  static constexpr int kElems = N, kSrcElem = sizeof(typename From::Elem),
+                       kDstElem = sizeof(typename To::Elem);
   static __device__ __forceinline__ Dst run(Src v) {
     typename From::Elem in[N];
     typename To::Elem out[N];
@@ -598,7 +621,16 @@ struct Cast {
   }
 };
 
-template <typename Op, int U, bool NT, typename Slots>
+// LOOSE: rows of at least one vector whose addresses or sizes are no multiples of it. Their
+// last vector starts `back` elements early, so that it ends with the row (the elements it
+// shares with the one before are written twice, with the same values), and every access
+// takes any address: what rows cost is an access and a slot per lane, whatever the width.
+// Measured on MI355X, 3,001 rows of 2 KiB in 64 arrays at multiples of 8, 4, 2 and 1 bytes:
+// in vectors of that width 177, 198, 479 and 781 us (row by row, with one slot a row: 141,
+// 147, 294 and 469), in 16 bytes at any address 138, 137, 161 and 160. float32 rows at
+// multiples of 4, rounded to bfloat16: an element a lane 371, so 209 (cast by torch first 333);
+// bfloat16 rows of 500 elements to e4m3 244, so 67 (107).
+template <typename Op, int U, bool NT, bool LOOSE, typename Slots>
 __device__ __forceinline__ void scatter_share(const PoolView& pool, int32_t layers,
                                               int32_t first_layer, int32_t n_layers,
                                               const char* k, const char* v, int64_t layer_stride,
@@ -613,45 +645,62 @@ __device__ __forceinline__ void scatter_share(const PoolView& pool, int32_t laye
   const uint32_t offset0 = base - row0 * sh.row_vecs;
   const bool is_v = y >= static_cast<uint32_t>(n_layers);
   const int32_t l = is_v ? y - n_layers : y;
-  const gptr<const Src> s = as_global<Src>((is_v ? v : k) + l * layer_stride) + base;
+  const char* s = (is_v ? v : k) + l * layer_stride;
   char* dst = array_base(pool, (is_v ? layers : 0) + first_layer + l);
-  const int64_t row_bytes = static_cast<int64_t>(sh.row_vecs) * sizeof(Dst);
+  const int64_t row_elems = static_cast<int64_t>(sh.row_vecs) * Op::kElems - sh.back;
   const uint32_t t = threadIdx.x;
   const uint32_t left = sh.vecs - base;   // > 0: the last workgroup may hold fewer
+  // The row (from row0) and, in elements, the place in it of vector u of this lane.
+  auto place = [&](int u, uint32_t* q) -> uint32_t {
+    const uint32_t o = offset0 + u * kThreads + t;
+    *q = o / sh.row_vecs;
+    const uint32_t j = o - *q * sh.row_vecs;
+    const uint32_t e = j * Op::kElems;
+    return LOOSE && j + 1 == static_cast<uint32_t>(sh.row_vecs) ? e - sh.back : e;
+  };
   Src r[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (u * kThreads + t < left) r[u] = load_vec<Src, NT>(s + u * kThreads + t);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     if (u * kThreads + t >= left) continue;
-    const uint32_t o = offset0 + u * kThreads + t;
-    const uint32_t q = o / sh.row_vecs;
+    if constexpr (LOOSE) {
+      uint32_t q;
+      const uint32_t e = place(u, &q);
+      r[u] = load_loose<Src, NT>(s + ((row0 + q) * row_elems + e) * Op::kSrcElem);
+    } else {
+      r[u] = load_vec<Src, NT>(as_global<Src>(s) + base + u * kThreads + t);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (u * kThreads + t >= left) continue;
+    uint32_t q;
+    const uint32_t e = place(u, &q);
     const int64_t slot = slots[row0 + q];
     if (slot < 0 || slot >= pool_rows) continue;   // never address outside the pool
-    store_vec<Dst, NT>(as_global<Dst>(dst + slot * row_bytes) + (o - q * sh.row_vecs),
-                       Op::run(r[u]));
+    char* d = dst + (slot * row_elems + e) * Op::kDstElem;
+    if constexpr (LOOSE) store_loose<Dst, NT>(d, Op::run(r[u]));
+    else store_vec<Dst, NT>(as_global<Dst>(d), Op::run(r[u]));
   }
 }
 
-template <typename Op, int U, bool NT>
+template <typename Op, int U, bool NT, bool LOOSE>
 __global__ void __launch_bounds__(kThreads)
 kv_scatter_rows(PoolView pool, int32_t layers, int32_t first_layer, int32_t n_layers,
                 const char* __restrict__ k, const char* __restrict__ v, int64_t layer_stride,
                 DeviceSlots slots, int64_t pool_rows, ScatterShape sh) {
-  scatter_share<Op, U, NT>(pool, layers, first_layer, n_layers, k, v, layer_stride, slots,
-                           pool_rows, sh);
+  scatter_share<Op, U, NT, LOOSE>(pool, layers, first_layer, n_layers, k, v, layer_stride, slots,
+                                  pool_rows, sh);
 }
 
 // The same with the slots in the kernel arguments (host slot lists): no upload
 // precedes the launch.
-template <typename Op, int U, bool NT, int W>
+template <typename Op, int U, bool NT, bool LOOSE, int W>
 __global__ void __launch_bounds__(kThreads)
 kv_scatter_inline(PoolView pool, int32_t layers, int32_t first_layer, int32_t n_layers,
                   const char* __restrict__ k, const char* __restrict__ v, int64_t layer_stride,
                   InlineSlots<W> slots, int64_t pool_rows, ScatterShape sh) {
-  scatter_share<Op, U, NT>(pool, layers, first_layer, n_layers, k, v, layer_stride, slots,
-                           pool_rows, sh);
+  scatter_share<Op, U, NT, LOOSE>(pool, layers, first_layer, n_layers, k, v, layer_stride, slots,
+                                  pool_rows, sh);
 }
 
 // gather_context over arrays: the context of array first_array + y is one run of
@@ -1559,19 +1608,27 @@ int check_write(const RowWrite& w, const int64_t* slots, int32_t n_tokens) {
 constexpr int kScatterU = 1;
 template <typename Op>
 constexpr int kCastU = sizeof(typename Op::Dst) <= 4 ? 4 : 1;
+// The same for rows at addresses that are no multiple of their vectors (LOOSE), with 1, 2
+// and 4: 3,001 rows of 2,048 bytes at multiples of 8 138 / 139 / 145 us, at odd addresses
+// 160 / 144 / 156; 3,000 rows of 1,000 bytes in 56 arrays 60 / 61 / 67, of 162 13 / 13 / 13.
+constexpr int kLooseU = 1;
+// And for rows of less than one vector (of 16 source bytes): 3,000 rows of 8 bytes in
+// 56 arrays, by random slots, 4.56 / 4.60 / 6.08, of 7 6.20 / 5.32 / 5.84.
+constexpr int kNarrowU = 2;
 // Slots one scatter launch carries in its arguments: a decode step's, and a longer
 // block (arguments cost the host per KiB, see InlineIds).
 constexpr int kSmallSlots = 64;
 constexpr int kLongSlots = IEKV_INLINE_IDS;
 
-// Launches a checked scatter whose rows are `row_vecs` vectors of Op::Src, in as many
-// launches as the slots in the arguments (host slots), 32-bit vector numbers and the
-// dispatch limit need (iekv_plan::cut_rows).
-template <typename Op, int U>
-int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t row_vecs,
+// Launches a checked scatter whose rows are `row_elems` elements of Op (at least one
+// vector of them), in as many launches as the slots in the arguments (host slots), 32-bit
+// vector numbers and the dispatch limit need (iekv_plan::cut_rows).
+template <typename Op, int U, bool LOOSE = false>
+int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t row_elems,
                     hipStream_t stream) {
   const int64_t per_group = kThreads * U;
   const int32_t layers = w.pool->n_arrays / 2;
+  const int64_t row_vecs = (row_elems + Op::kElems - 1) / Op::kElems;
   const iekv_plan::RowCut cut = iekv_plan::cut_rows(
       row_vecs, w.n_layers, per_group, list.on_host ? kLongSlots : INT32_MAX, kMaxGrid / 2);
   DeviceGuard guard(w.pool->device);
@@ -1583,12 +1640,12 @@ int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t 
   auto launch = [&](int64_t first, int32_t n, int32_t l0, int32_t n_layers) -> int {
     ScatterShape sh;
     sh.row_vecs = static_cast<int32_t>(row_vecs);
+    sh.back = static_cast<int32_t>(row_vecs * Op::kElems - row_elems);
     sh.vecs = static_cast<int32_t>(n * row_vecs);
     sh.chunks = static_cast<int32_t>((sh.vecs + per_group - 1) / per_group);
     sh.xcd = (g_order.load() & iekv_plan::kXcdGrouped) != 0 ? 1 : 0;
     sh.groups = sh.chunks * 2 * n_layers;
-    const int64_t skip = l0 * w.layer_stride +
-                         first * row_vecs * static_cast<int64_t>(sizeof(typename Op::Src));
+    const int64_t skip = l0 * w.layer_stride + first * row_elems * Op::kSrcElem;
     auto go = [&](auto kernel, const auto& slots) {
       return dispatch(kernel, dim3(static_cast<uint32_t>(sh.groups)), stream, view, layers,
                       w.first_layer + l0, n_layers, w.k + skip, w.v + skip, w.layer_stride, slots,
@@ -1598,13 +1655,13 @@ int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t 
       constexpr int W = decltype(words)::value;
       InlineSlots<W> slots{};
       std::copy(list.slots + first, list.slots + first + n, slots.slots);
-      return nt ? go(kv_scatter_inline<Op, U, true, W>, slots)
-                : go(kv_scatter_inline<Op, U, false, W>, slots);
+      return nt ? go(kv_scatter_inline<Op, U, true, LOOSE, W>, slots)
+                : go(kv_scatter_inline<Op, U, false, LOOSE, W>, slots);
     };
     if (!list.on_host) {
       const DeviceSlots slots{list.slots + first};
-      return nt ? go(kv_scatter_rows<Op, U, true>, slots)
-                : go(kv_scatter_rows<Op, U, false>, slots);
+      return nt ? go(kv_scatter_rows<Op, U, true, LOOSE>, slots)
+                : go(kv_scatter_rows<Op, U, false, LOOSE>, slots);
     }
     return n <= kSmallSlots ? inlined(std::integral_constant<int, kSmallSlots>{})
                             : inlined(std::integral_constant<int, kLongSlots>{});
@@ -1618,17 +1675,20 @@ int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t 
   return IEKV_OK;
 }
 
-// A cast, 16 source bytes a lane where the rows allow it, else one element.
+// A cast: 16 source bytes a lane, at any address where the rows do not keep them aligned;
+// rows of fewer elements than that one element a lane.
 template <typename From, typename To>
 int launch_cast(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t row_elems, int align,
                 hipStream_t stream) {
   constexpr int kWide = 16 / sizeof(typename From::Elem);
   using Wide = Cast<From, To, kWide>;
-  // Both rows hold whole vectors, and both sides' addresses are multiples of them.
+  if (row_elems < kWide)
+    return launch_write_as<Cast<From, To, 1>, kNarrowU>(w, list, n_tokens, row_elems, stream);
+  // Aligned: both rows hold whole vectors, and both sides' addresses are multiples of them.
   if (align == 16 && row_elems % kWide == 0 &&
       w.pool->align >= static_cast<int>(sizeof(typename Wide::Dst)))
-    return launch_write_as<Wide, kCastU<Wide>>(w, list, n_tokens, row_elems / kWide, stream);
-  return launch_write_as<Cast<From, To, 1>, 4>(w, list, n_tokens, row_elems, stream);
+    return launch_write_as<Wide, kCastU<Wide>>(w, list, n_tokens, row_elems, stream);
+  return launch_write_as<Wide, kLooseU, true>(w, list, n_tokens, row_elems, stream);
 }
 
 // A checked scatter of n_tokens >= 1 rows.
@@ -1651,14 +1711,15 @@ int launch_write(const RowWrite& w, SlotList list, int32_t n_tokens, hipStream_t
     return launch_cast<FromBf16, ToE4m3>(w, list, n_tokens, elems, align, stream);
   }
   align = std::min({align, w.pool->align, align_of_ptr(static_cast<uint64_t>(row_bytes))});
-  const int64_t row_vecs = row_bytes / align;
+  if (align == 16)
+    return launch_write_as<Bytes<u32x4>, kScatterU>(w, list, n_tokens, row_bytes, stream);
+  if (row_bytes >= 16)
+    return launch_write_as<Bytes<u32x4>, kLooseU, true>(w, list, n_tokens, row_bytes, stream);
   switch (align) {
-    case 16:
-      return launch_write_as<Bytes<u32x4>, kScatterU>(w, list, n_tokens, row_vecs, stream);
-    case 8: return launch_write_as<Bytes<u32x2>, 4>(w, list, n_tokens, row_vecs, stream);
-    case 4: return launch_write_as<Bytes<uint32_t>, 4>(w, list, n_tokens, row_vecs, stream);
-    case 2: return launch_write_as<Bytes<uint16_t>, 4>(w, list, n_tokens, row_vecs, stream);
-    default: return launch_write_as<Bytes<uint8_t>, 4>(w, list, n_tokens, row_vecs, stream);
+    case 8: return launch_write_as<Bytes<u32x2>, kNarrowU>(w, list, n_tokens, row_bytes, stream);
+    case 4: return launch_write_as<Bytes<uint32_t>, kNarrowU>(w, list, n_tokens, row_bytes, stream);
+    case 2: return launch_write_as<Bytes<uint16_t>, kNarrowU>(w, list, n_tokens, row_bytes, stream);
+    default: return launch_write_as<Bytes<uint8_t>, kNarrowU>(w, list, n_tokens, row_bytes, stream);
   }
 }
 

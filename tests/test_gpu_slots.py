@@ -363,3 +363,67 @@ def test_captured_writes_replay_and_uploads_are_refused_under_capture(gpu):
         torch.cuda.synchronize()
         assert all(torch.equal(w.view(torch.int16), c.view(torch.int16))
                    for w, c in zip(want, k + v)), step      # bytes: the pool holds NaNs
+
+
+@pytest.mark.parametrize("row", [1, 2, 7, 8, 12, 15, 16, 17, 24, 31, 33, 162, 1000, 2056])
+@pytest.mark.parametrize("offset", [0, 1, 2, 4, 8])
+def test_rows_of_any_size_at_any_address_are_written(gpu, row, offset):
+    """Rows of bytes on either side of one 16-byte vector, whole ones and not, at addresses
+    that are multiples of 16, 8, 4, 2 and 1: every row lands in its slot, the bytes of the
+    other slots stay, and so do those beside the arrays."""
+    from iekv.engine.pools import KVPool, allocate_pool
+    from iekv.engine.slots import write_slots_layers
+
+    for n in (1, 16, 257, 600):
+        k, v = allocate_pool(41, 16, 2, 1, row, dtype=torch.uint8, device=gpu, zero=False,
+                             pad_blocks=1)
+        slab = k[0]._base
+        slab.random_(0, 256, generator=torch.Generator(gpu).manual_seed(n))
+        pool = KVPool(k, v, 16)
+        total = 2 * n * row
+        flat = torch.randint(0, 256, (2 * total + 32,), dtype=torch.uint8, device=gpu,
+                             generator=torch.Generator(gpu).manual_seed(row))
+        rows_k = flat[offset:offset + total].view(2, n, 1, row)
+        rows_v = flat[total + 16:2 * total + 16].view(2, n, 1, row)
+        where = torch.from_numpy(np.random.default_rng(n + row).permutation(41 * 16)[:n]).to(gpu)
+        want = slab.clone()
+        for l in range(2):
+            want[0, l, where] = rows_k[l]
+            want[1, l, where] = rows_v[l]
+        write_slots_layers(pool, rows_k, rows_v, where if n != 257 else where.tolist())
+        assert torch.equal(slab, want), n
+
+
+@pytest.mark.parametrize("elems", [3, 4, 5, 7, 8, 9, 15, 27, 125, 256])
+@pytest.mark.parametrize("row_dtype,cache_dtype", [
+    (torch.float32, torch.float16), (torch.float32, torch.bfloat16),
+    (torch.float32, torch.float8_e4m3fn), (torch.float16, torch.float8_e4m3fn),
+    (torch.bfloat16, torch.float8_e4m3fn)], ids=str)
+def test_casts_of_any_row_size_at_any_address(gpu, elems, row_dtype, cache_dtype):
+    """Rows of another type on either side of one vector's elements, whole vectors and not,
+    aligned and one element in, with one launch and several (host lists over 256 slots),
+    an upload and device slots: each equals torch's cast, and nothing else changes."""
+    from iekv.engine.pools import KVPool, allocate_pool
+    from iekv.engine.slots import write_slots_layers
+
+    for n in (1, 65, 257, 513):
+        for first in (0, 1):
+            k, v = allocate_pool(66, 8, 2, 1, elems, dtype=cache_dtype, device=gpu, zero=False,
+                                 pad_blocks=1)
+            slab = k[0]._base.view(torch.uint8)
+            slab.random_(0, 256, generator=torch.Generator(gpu).manual_seed(n))
+            pool = KVPool(k, v, 8)
+            total = 2 * n * elems
+            pad = -total % 16 + 16
+            flat = (torch.randn(2 * total + 2 * pad, device=gpu,
+                                generator=torch.Generator(gpu).manual_seed(elems)) * 50
+                    ).to(row_dtype)
+            rows_k = flat[first:first + total].view(2, n, 1, elems)
+            rows_v = flat[total + pad:2 * total + pad].view(2, n, 1, elems)
+            where = torch.from_numpy(np.random.default_rng(n).permutation(66 * 8)[:n]).to(gpu)
+            want = slab.clone()
+            for l in range(2):
+                want[0, l, where] = rows_k[l].to(cache_dtype).view(torch.uint8)
+                want[1, l, where] = rows_v[l].to(cache_dtype).view(torch.uint8)
+            write_slots_layers(pool, rows_k, rows_v, where if n == 65 else where.tolist())
+            assert torch.equal(slab, want), (n, first)
