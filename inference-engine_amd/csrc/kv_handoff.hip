@@ -714,6 +714,9 @@ kv_scatter_inline(PoolView pool, int32_t layers, int32_t first_layer, int32_t n_
 // per array. It is bound by HBM: scattered 32 KiB reads against streaming writes.
 struct GatherShape {
   int32_t tile_vecs;   // vectors per block
+  int32_t tile_bytes;  // of a block, and of the used part of block last_block (LOOSE only)
+  int32_t last_bytes;
+  uint32_t last_block;
   int32_t vecs;        // vectors per array in this launch (host: fits int32)
   int32_t chunks;      // workgroups per array
   int32_t xcd;         // 1: XCD-grouped workgroup positions
@@ -734,23 +737,36 @@ struct InlineTable {
 // SPANS: a workgroup's vectors may lie in several blocks (kThreads * U does not
 // divide tile_vecs), so each lane finds its own; otherwise the block, and its
 // table entry, are the same for the whole workgroup and read with scalar loads.
-template <typename V, int U, bool NT, bool SPANS, typename Table>
+// LOOSE (with SPANS, and 16 bytes or more of every block): blocks, contexts or the output
+// whose sizes or addresses are no multiples of a vector. A block's last vector ends with its
+// used bytes (those it shares with the one before are written twice, the same), and every
+// access takes any address, as in the scatter. Measured on MI355X, 3,001 tokens, row by row /
+// in vectors of what divides them, four a lane / so, us: 56 arrays, rows of 1,000 bytes
+// 57.1 / 80.5 / 56.8, of 2,056 134 / 163 / 114, of 162 52 / 38 / 12, of 24 5.3 / 6.1 / 4.3;
+// 64 arrays of 2 KiB rows, output at multiples of 8, 4, 2 and 1 bytes 136 / 137 / 127,
+// 158 / 160 / 127, 279 / 358 / 133, 453 / 678 / 133. Two vectors a lane are level, four 1-25%
+// slower.
+template <typename V, int U, bool NT, bool SPANS, bool LOOSE, typename Table>
 __device__ __forceinline__ void gather_share(const PoolView& pool, int32_t first_array,
                                              const Table& table, char* out, int64_t out_stride,
                                              const GatherShape& sh) {
+  static_assert(SPANS || !LOOSE, "a lane finds its block's last vector by its own division");
   const uint32_t w = sh.xcd ? iekv_plan::xcd_grouped(blockIdx.x, sh.groups) : blockIdx.x;
   const uint32_t y = w / sh.chunks;
   const uint32_t base = (w - y * sh.chunks) * (kThreads * U);
   const uint32_t block0 = base / sh.tile_vecs;
   const uint32_t offset0 = base - block0 * sh.tile_vecs;
   const char* src = array_base(pool, first_array + y);
-  const int64_t tile_bytes = static_cast<int64_t>(sh.tile_vecs) * sizeof(V);
+  const int64_t tile_bytes =
+      LOOSE ? sh.tile_bytes : static_cast<int64_t>(sh.tile_vecs) * sizeof(V);
   const uint32_t t = threadIdx.x;
   const uint32_t left = sh.vecs - base;   // > 0: the last workgroup may hold fewer
-  const RunOut<V, NT, true> d(as_global<V>(out + y * out_stride) + base,
+  char* to = out + y * out_stride;
+  const RunOut<V, NT, !LOOSE> d(as_global<V>(to) + base,
                                 min(left, static_cast<uint32_t>(kThreads * U)));
   V v[U];
   bool have[U];
+  int64_t at[U];   // LOOSE: where the vector goes
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     uint32_t o = offset0 + u * kThreads + t;
@@ -764,28 +780,39 @@ __device__ __forceinline__ void gather_share(const PoolView& pool, int32_t first
     if (have[u]) {
       const int32_t id = table[block];
       have[u] = id >= 0 && id < pool.num_blocks;   // never address outside the pool
-      if (have[u]) v[u] = load_vec<V, NT>(as_global<V>(src + id * tile_bytes) + o);
+      if constexpr (LOOSE) {
+        const uint32_t size = block == sh.last_block ? sh.last_bytes : sh.tile_bytes;
+        const uint32_t in_block = min(o * static_cast<uint32_t>(sizeof(V)),
+                                      size - static_cast<uint32_t>(sizeof(V)));
+        at[u] = block * tile_bytes + in_block;
+        if (have[u]) v[u] = load_loose<V, NT>(src + id * tile_bytes + in_block);
+      } else {
+        if (have[u]) v[u] = load_vec<V, NT>(as_global<V>(src + id * tile_bytes) + o);
+      }
     }
   }
 #pragma unroll
-  for (int u = 0; u < U; ++u)
-    if (have[u]) d.store(u * kThreads + t, v[u]);
+  for (int u = 0; u < U; ++u) {
+    if (!have[u]) continue;
+    if constexpr (LOOSE) store_loose<V, NT>(to + at[u], v[u]);
+    else d.store(u * kThreads + t, v[u]);
+  }
 }
 
-template <typename V, int U, bool NT, bool SPANS>
+template <typename V, int U, bool NT, bool SPANS, bool LOOSE>
 __global__ void __launch_bounds__(kThreads)
 kv_gather_rows(PoolView pool, int32_t first_array, DeviceTable table, char* __restrict__ out,
                int64_t out_stride, GatherShape sh) {
-  gather_share<V, U, NT, SPANS>(pool, first_array, table, out, out_stride, sh);
+  gather_share<V, U, NT, SPANS, LOOSE>(pool, first_array, table, out, out_stride, sh);
 }
 
 // The same with the table in the kernel arguments (host block tables): no upload
 // precedes the launch.
-template <typename V, int U, bool NT, bool SPANS, int W>
+template <typename V, int U, bool NT, bool SPANS, bool LOOSE, int W>
 __global__ void __launch_bounds__(kThreads)
 kv_gather_inline(PoolView pool, int32_t first_array, InlineTable<W> table,
                  char* __restrict__ out, int64_t out_stride, GatherShape sh) {
-  gather_share<V, U, NT, SPANS>(pool, first_array, table, out, out_stride, sh);
+  gather_share<V, U, NT, SPANS, LOOSE>(pool, first_array, table, out, out_stride, sh);
 }
 
 // Block-id checks of iekv_check_ids, three launches in stream order: clear the
@@ -1762,11 +1789,11 @@ int check_gather(const iekv_pool* pool, int32_t first_array, int32_t n_arrays,
 
 // One launch of a checked gather: `vecs` vectors of V per array, out of the blocks
 // of table[0 ..] (device memory, or `count` host ids for the arguments).
-template <typename V, int U>
+template <typename V, int U, bool LOOSE = false>
 int launch_gather_as(const iekv_pool* pool, int32_t first_array, GatherShape sh, IdList table,
                      int32_t count, char* out, int64_t out_stride, hipStream_t stream) {
   const bool nt = g_nontemporal.load() != 0;
-  const bool spans = sh.tile_vecs % (kThreads * U) != 0;
+  const bool spans = LOOSE || sh.tile_vecs % (kThreads * U) != 0;
   const PoolView view = view_of(pool);
   const dim3 grid(static_cast<uint32_t>(sh.groups));
   auto inlined = [&](auto words) {
@@ -1776,10 +1803,10 @@ int launch_gather_as(const iekv_pool* pool, int32_t first_array, GatherShape sh,
     auto go = [&](auto kernel) {
       return dispatch(kernel, grid, stream, view, first_array, t, out, out_stride, sh);
     };
-    if (nt) return spans ? go(kv_gather_inline<V, U, true, true, W>)
-                         : go(kv_gather_inline<V, U, true, false, W>);
-    return spans ? go(kv_gather_inline<V, U, false, true, W>)
-                 : go(kv_gather_inline<V, U, false, false, W>);
+    if (spans) return nt ? go(kv_gather_inline<V, U, true, true, LOOSE, W>)
+                         : go(kv_gather_inline<V, U, false, true, LOOSE, W>);
+    return nt ? go(kv_gather_inline<V, U, true, false, false, W>)
+              : go(kv_gather_inline<V, U, false, false, false, W>);
   };
   if (table.on_host)
     return count <= kSmallTable ? inlined(std::integral_constant<int, kSmallTable>{})
@@ -1788,9 +1815,10 @@ int launch_gather_as(const iekv_pool* pool, int32_t first_array, GatherShape sh,
   auto go = [&](auto kernel) {
     return dispatch(kernel, grid, stream, view, first_array, t, out, out_stride, sh);
   };
-  if (nt) return spans ? go(kv_gather_rows<V, U, true, true>)
-                       : go(kv_gather_rows<V, U, true, false>);
-  return spans ? go(kv_gather_rows<V, U, false, true>) : go(kv_gather_rows<V, U, false, false>);
+  if (spans) return nt ? go(kv_gather_rows<V, U, true, true, LOOSE>)
+                       : go(kv_gather_rows<V, U, false, true, LOOSE>);
+  return nt ? go(kv_gather_rows<V, U, true, false, false>)
+            : go(kv_gather_rows<V, U, false, false, false>);
 }
 
 // A checked gather of context_len >= 1 rows of n_arrays arrays, in launches of as
@@ -1805,27 +1833,35 @@ int launch_gather(const iekv_pool* pool, int32_t first_array, int32_t n_arrays,
   // arrays' contexts allow.
   int vec = std::min(pool->align, align_of_ptr(reinterpret_cast<uint64_t>(out)));
   vec = std::min(vec, align_of_ptr(static_cast<uint64_t>(out_stride)));
-  const int64_t tile_vecs = pool->tile_bytes / vec;
+  const int64_t blocks = (static_cast<int64_t>(context_len) - 1) / block_size + 1;
+  const int64_t last_bytes = out_stride - (blocks - 1) * pool->tile_bytes;
+  // Where they are no multiples of 16 bytes but every block holds as many, vectors of 16 at
+  // any address.
+  const bool loose = vec < 16 && std::min(pool->tile_bytes, last_bytes) >= 16;
+  if (loose) vec = 16;
+  const int64_t tile_vecs = (pool->tile_bytes + vec - 1) / vec;
   const int64_t per_group = kThreads * (vec == 16 ? kGatherU : 4);
   const iekv_plan::RowCut cut = iekv_plan::cut_rows(
       tile_vecs, n_arrays, per_group, table.on_host ? kLongTable : INT32_MAX, kMaxGrid);
-  const int64_t blocks = (static_cast<int64_t>(context_len) - 1) / block_size + 1;
   DeviceGuard guard(pool->device);
   if (!guard.ok()) return guard.fail();
   // One launch: blocks first .. first + count - 1 of arrays a0 .. a0 + arrays - 1 of the call.
   auto launch = [&](int64_t first, int32_t count, int32_t a0, int32_t arrays) -> int {
-    const int64_t begin = first * pool->tile_bytes;
-    const int64_t end = std::min((first + count) * pool->tile_bytes, out_stride);
+    const int64_t bytes = first + count < blocks ? pool->tile_bytes : last_bytes;
     GatherShape sh;
     sh.tile_vecs = static_cast<int32_t>(tile_vecs);
-    sh.vecs = static_cast<int32_t>((end - begin) / vec);
+    sh.tile_bytes = static_cast<int32_t>(pool->tile_bytes);
+    sh.last_bytes = static_cast<int32_t>(bytes);
+    sh.last_block = static_cast<uint32_t>(count - 1);
+    sh.vecs = static_cast<int32_t>((count - 1) * tile_vecs + (bytes + vec - 1) / vec);
     sh.chunks = static_cast<int32_t>((sh.vecs + per_group - 1) / per_group);
     sh.xcd = (g_pack_order.load() & iekv_plan::kXcdGrouped) != 0 ? 1 : 0;
     sh.groups = sh.chunks * arrays;
-    char* to = out + a0 * out_stride + begin;
+    char* to = out + a0 * out_stride + first * pool->tile_bytes;
     auto go = [&](auto kernel) {
       return kernel(pool, first_array + a0, sh, table.from(first), count, to, out_stride, stream);
     };
+    if (loose) return go(launch_gather_as<u32x4, kGatherU, true>);
     switch (vec) {
       case 16: return go(launch_gather_as<u32x4, kGatherU>);
       case 8: return go(launch_gather_as<u32x2, 4>);

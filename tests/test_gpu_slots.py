@@ -427,3 +427,34 @@ def test_casts_of_any_row_size_at_any_address(gpu, elems, row_dtype, cache_dtype
                 want[1, l, where] = rows_v[l].to(cache_dtype).view(torch.uint8)
             write_slots_layers(pool, rows_k, rows_v, where if n == 65 else where.tolist())
             assert torch.equal(slab, want), (n, first)
+
+
+@pytest.mark.parametrize("row", [1, 3, 7, 8, 12, 15, 16, 17, 24, 31, 162, 1000, 2056])
+@pytest.mark.parametrize("offset", [0, 1, 8])
+def test_contexts_of_any_row_size_are_gathered_to_any_address(gpu, row, offset):
+    """Contexts of blocks on either side of one 16-byte vector, whole ones and not, last
+    blocks of one row and of all, into outputs at multiples of 16, 8 and 1 bytes, by host
+    and by device tables: every byte of every context, and none beside them."""
+    from iekv import _native
+    from iekv.engine.pools import KVPool, allocate_pool, current_stream_handle
+
+    for bs in (1, 5, 16):
+        k, v = allocate_pool(530, bs, 2, 1, row, dtype=torch.uint8, device=gpu, zero=False)
+        k[0]._base.random_(0, 256, generator=torch.Generator(gpu).manual_seed(bs))
+        pool = KVPool(k, v, bs)
+        table = [int(b) for b in np.random.default_rng(row).permutation(530)]
+        on_device = torch.tensor(table, dtype=torch.int32, device=gpu)
+        on_host = np.array(table, np.int32)
+        rows = (on_device.long()[:, None] * bs + torch.arange(bs, device=gpu)).reshape(-1)
+        for tokens in {1, bs, bs + 1, 37 * bs, 514 * bs - bs // 2}:
+            want = torch.stack([c[rows[:tokens]] for c in k + v]).view(torch.uint8).reshape(-1)
+            for fn, address in (("iekv_gather_rows_arrays", on_device.data_ptr()),
+                                ("iekv_gather_rows_arrays_ids", on_host.ctypes.data)):
+                out = torch.full((want.numel() + 512,), 0xA5, dtype=torch.uint8, device=gpu)
+                _native.call(fn, pool.native.handle, 0, 4, bs, address, tokens,
+                             out.data_ptr() + 256 + offset, want.numel(),
+                             current_stream_handle(pool.device))
+                at = 256 + offset
+                assert torch.equal(out[at:at + want.numel()], want), (bs, tokens, fn)
+                assert bool((out[:at] == 0xA5).all()) and \
+                    bool((out[at + want.numel():] == 0xA5).all()), (bs, tokens, fn)
