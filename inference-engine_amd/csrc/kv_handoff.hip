@@ -519,12 +519,17 @@ constexpr int kWave = 64;
 // layers + first_layer + l). Array index y of the launch is K of layer y for
 // y < n_layers, then V. A layer's rows are one run of bytes, so the scatter works in
 // vectors of that run, kThreads * U per workgroup, whatever the row size: a vector's
-// row is its number / row_vecs, and every lane has one (see the gather below).
+// row is its number / row_vecs, and every lane has one (see the gather below). The division
+// is a shift where it can be: a lane has one vector's traffic to hide some 30 instructions
+// behind. Measured on MI355X, division / shift / row by row: 150 rows of 2 KiB in 64 arrays
+// 9.5 / 8.6 / 9.2 us, 3,000 of 256 bytes in 48 15.1 / 13.7 / 14.2, 300 of 1 KiB in 160
+// 19.4 / 18.6 / 19.0, 3,001 of 2 KiB in 64 level.
 // The source vectors are loaded before the slots are read, so the two latencies
 // overlap (the 70B-shape share's 1 KiB rows ran at 6.13-6.30 TB/s that way, 5.47-5.57
 // with the slot read first).
 struct ScatterShape {
   int32_t row_vecs;   // source vectors per row
+  int32_t row_shift;  // its logarithm where it is a power of two, else -1
   int32_t back;       // elements a row's last vector starts before the end of the one before it
   int32_t vecs;       // source vectors per layer in this launch (host: fits int32)
   int32_t chunks;     // workgroups per array
@@ -653,7 +658,7 @@ __device__ __forceinline__ void scatter_share(const PoolView& pool, int32_t laye
   // The row (from row0) and, in elements, the place in it of vector u of this lane.
   auto place = [&](int u, uint32_t* q) -> uint32_t {
     const uint32_t o = offset0 + u * kThreads + t;
-    *q = o / sh.row_vecs;
+    *q = sh.row_shift >= 0 ? o >> sh.row_shift : o / sh.row_vecs;
     const uint32_t j = o - *q * sh.row_vecs;
     const uint32_t e = j * Op::kElems;
     return LOOSE && j + 1 == static_cast<uint32_t>(sh.row_vecs) ? e - sh.back : e;
@@ -1633,6 +1638,13 @@ int check_write(const RowWrite& w, const int64_t* slots, int32_t n_tokens) {
 // by torch first: 330); 70B share, 8,000 bfloat16 rows to e4m3 688 / 719 / 716 (torch
 // first: 1,083), 3,000 float32 rows to e4m3 477 / 442 / 404 (torch first: 580).
 constexpr int kScatterU = 1;
+// Except launches of more workgroups than the GPU's 256 compute units hold at once (8 each)
+// and not quite twice as many: two vectors a lane leave no second, mostly empty turn. With
+// 1 / 2, row by row: 3,001 rows of 2 KiB in 2 arrays (3,002 workgroups of one vector)
+// 5.8 / 5.4, 5.6 us; 100 in 64 (3,200) 6.1 / 5.8, 6.4; 64 of 1 KiB in 160 (2,560) 5.3 / 5.2,
+// 5.8; but 150 in 64 (4,800) 8.6 / 9.6, 9.2, and 3,000 of 16 bytes in 56 arrays, by random
+// slots (672), 5.2 / 5.7, 5.2.
+constexpr int64_t kScatterTwoLeast = 2049, kScatterTwoMost = 3584;
 template <typename Op>
 constexpr int kCastU = sizeof(typename Op::Dst) <= 4 ? 4 : 1;
 // The same for rows at addresses that are no multiple of their vectors (LOOSE), with 1, 2
@@ -1667,6 +1679,7 @@ int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t 
   auto launch = [&](int64_t first, int32_t n, int32_t l0, int32_t n_layers) -> int {
     ScatterShape sh;
     sh.row_vecs = static_cast<int32_t>(row_vecs);
+    sh.row_shift = row_vecs & (row_vecs - 1) ? -1 : __builtin_ctzll(row_vecs);
     sh.back = static_cast<int32_t>(row_vecs * Op::kElems - row_elems);
     sh.vecs = static_cast<int32_t>(n * row_vecs);
     sh.chunks = static_cast<int32_t>((sh.vecs + per_group - 1) / per_group);
@@ -1738,8 +1751,12 @@ int launch_write(const RowWrite& w, SlotList list, int32_t n_tokens, hipStream_t
     return launch_cast<FromBf16, ToE4m3>(w, list, n_tokens, elems, align, stream);
   }
   align = std::min({align, w.pool->align, align_of_ptr(static_cast<uint64_t>(row_bytes))});
-  if (align == 16)
+  if (align == 16) {
+    const int64_t groups = (n_tokens * (row_bytes / 16) + kThreads - 1) / kThreads * 2 * w.n_layers;
+    if (groups >= kScatterTwoLeast && groups <= kScatterTwoMost)
+      return launch_write_as<Bytes<u32x4>, 2>(w, list, n_tokens, row_bytes, stream);
     return launch_write_as<Bytes<u32x4>, kScatterU>(w, list, n_tokens, row_bytes, stream);
+  }
   if (row_bytes >= 16)
     return launch_write_as<Bytes<u32x4>, kLooseU, true>(w, list, n_tokens, row_bytes, stream);
   switch (align) {

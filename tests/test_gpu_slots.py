@@ -458,3 +458,20 @@ def test_contexts_of_any_row_size_are_gathered_to_any_address(gpu, row, offset):
                 assert torch.equal(out[at:at + want.numel()], want), (bs, tokens, fn)
                 assert bool((out[:at] == 0xA5).all()) and \
                     bool((out[at + want.numel():] == 0xA5).all()), (bs, tokens, fn)
+
+
+@pytest.mark.parametrize("n", [2047, 2048, 2049, 3584, 3585])
+def test_writes_of_one_and_of_two_vectors_a_lane(gpu, n):
+    """Aligned rows of one layer around the launch sizes that take two vectors a lane, rows
+    of a power of two of vectors and not."""
+    from iekv.engine.slots import write_slots
+
+    for dim in (2048, 2064):        # 128 and 129 vectors a row
+        k, v, pool = random_pool(230, 16, 1, dim, torch.uint8, gpu, layers=1, seed=n)
+        rows = torch.randint(0, 256, (2, n, 1, dim), dtype=torch.uint8, device=gpu,
+                             generator=torch.Generator(gpu).manual_seed(dim))
+        where = torch.from_numpy(np.random.default_rng(n).permutation(230 * 16)[:n]).to(gpu)
+        want = [c.clone() for c in k + v]
+        want[0][where], want[1][where] = rows[0], rows[1]
+        write_slots(pool, 0, rows[0], rows[1], where)
+        assert all(torch.equal(w, c) for w, c in zip(want, k + v)), dim
