@@ -27,12 +27,27 @@ from .pools import KVPool, current_stream_handle
 # tokens each): two launches. Longer lists are uploaded once.
 HOST_SLOTS_MAX = 2 * _native.INLINE_IDS
 
+# Longest host block table the library carries in its launches' arguments (512 entries each):
+# four launches. A longer one is uploaded and gathered in one: each launch more drains and
+# fills the GPU again. Host table / uploaded, whole call on MI355X, us: 1,024 blocks of 8
+# arrays of 8 KiB tiles 29 / 47, of 48 of 4 KiB 71 / 68; 2,048 53 / 66 and 152 / 140, of 64 of
+# 32 KiB 1,357 / 1,386; 4,096 103 / 105, 294 / 271 and 2,732 / 2,806; 8,192 of 8 arrays
+# 239 / 223, of 48 of 2 KiB 363 / 307 (row by row, uploaded, 240 and 317).
+HOST_TABLE_MAX = 2048
+
 _TYPES = {torch.float32: _native.IEKV_TYPE_F32, torch.float16: _native.IEKV_TYPE_F16,
           torch.bfloat16: _native.IEKV_TYPE_BF16, torch.float8_e4m3fn: _native.IEKV_TYPE_E4M3}
 # (row type, cache type) pairs iekv_write_slots_cast rounds on the way.
 _CASTS = {(torch.float32, torch.float16), (torch.float32, torch.bfloat16),
           (torch.float32, torch.float8_e4m3fn), (torch.float16, torch.float8_e4m3fn),
           (torch.bfloat16, torch.float8_e4m3fn)}
+
+
+def _capturing(device: torch.device) -> bool:
+    """Whether the device's current stream is under capture. An upload made there would be
+    replayed from its pinned source long after that was freed."""
+    with torch.cuda.device(device):
+        return torch.cuda.is_current_stream_capturing()
 
 
 def _slots(pool: KVPool, slots):
@@ -57,12 +72,10 @@ def _slots(pool: KVPool, slots):
     if checked.min() < 0 or checked.max() >= rows:
         bad = checked[(checked < 0) | (checked >= rows)][0]
         raise IndexError(f"slot {bad} out of range for a pool of {rows} slots")
-    with torch.cuda.device(pool.device):
-        if torch.cuda.is_current_stream_capturing():
-            # A replay would read the pinned copy of the list again, long after it was freed.
-            raise RuntimeError(f"a list of {len(host)} slots is uploaded, which a stream under "
-                               f"capture cannot do: pass a device tensor, or at most "
-                               f"{HOST_SLOTS_MAX} slots")
+    if _capturing(pool.device):
+        raise RuntimeError(f"a list of {len(host)} slots is uploaded, which a stream under "
+                           f"capture cannot do: pass a device tensor, or at most "
+                           f"{HOST_SLOTS_MAX} slots")
     t = torch.from_numpy(checked).pin_memory().to(pool.device, non_blocking=True)
     return t, "iekv_write_slots_cast"
 
@@ -111,7 +124,8 @@ def write_slots(pool: KVPool, layer: int, k: torch.Tensor, v: torch.Tensor, slot
 def _context_table(pool: KVPool, block_table, context_len: int):
     """The table entries a context uses, and the entry point that takes them: a device
     int32 tensor as it is, host ids as an int32 array the library checks and carries in
-    its launch (no upload). IndexError for a table too short for the context."""
+    its launches (no upload), long ones checked and uploaded. IndexError for a table too
+    short for the context."""
     needed = -(-context_len // pool.block_size)
     if isinstance(block_table, torch.Tensor):
         table = block_table.to(dtype=torch.int32)
@@ -122,6 +136,9 @@ def _context_table(pool: KVPool, block_table, context_len: int):
     if needed > len(block_table):
         raise IndexError(f"context of {context_len} needs {needed} blocks, table has "
                          f"{len(block_table)}")
+    if needed > HOST_TABLE_MAX and not _capturing(pool.device):
+        return pool.block_ids(block_table[:needed], what="context block"), \
+            "iekv_gather_rows_arrays"
     used = list(block_table[:needed])
     try:
         return _ints("i", used), "iekv_gather_rows_arrays_ids"

@@ -475,3 +475,26 @@ def test_writes_of_one_and_of_two_vectors_a_lane(gpu, n):
         want[0][where], want[1][where] = rows[0], rows[1]
         write_slots(pool, 0, rows[0], rows[1], where)
         assert all(torch.equal(w, c) for w, c in zip(want, k + v)), dim
+
+
+@pytest.mark.parametrize("blocks", [2047, 2048, 2049, 5000])
+def test_long_host_tables_gather_like_device_tables(gpu, blocks):
+    """Tables on either side of the longest that rides in launch arguments, as lists and
+    arrays: the rows a device table gives; ids outside the pool are refused either way."""
+    from iekv.engine.slots import gather_rows, gather_rows_arrays
+
+    k, v, pool = random_pool(5003, 3, 2, 20, torch.float16, gpu, layers=2, seed=blocks)
+    table = np.random.default_rng(blocks).permutation(5003)[:blocks]
+    on_device = torch.from_numpy(table.astype(np.int32)).to(gpu)
+    for context in (blocks * 3, blocks * 3 - 2):
+        want = gather_rows_arrays(pool, on_device, context).view(torch.uint8)
+        rows = (on_device.long()[:, None] * 3 + torch.arange(3, device=gpu)).reshape(-1)[:context]
+        assert torch.equal(want[0], k[0][rows].view(torch.uint8))
+        for form in (table.tolist(), table, tuple(table.tolist())):
+            assert torch.equal(gather_rows_arrays(pool, form, context).view(torch.uint8), want)
+            assert torch.equal(gather_rows(pool, 3, form, context).view(torch.uint8), want[3])
+    for bad in (-1, 5003):
+        with pytest.raises(IndexError, match="context block id"):
+            gather_rows_arrays(pool, table[:-1].tolist() + [bad], blocks * 3)
+    with pytest.raises(TypeError):
+        gather_rows_arrays(pool, table[:-1].tolist() + [1.5], blocks * 3)

@@ -2,6 +2,7 @@
 from contextlib import nullcontext
 from types import SimpleNamespace
 
+import numpy as np
 import pytest
 import torch
 
@@ -22,3 +23,25 @@ def test_a_list_that_would_be_uploaded_is_refused_under_capture(monkeypatch):
     with pytest.raises(IndexError, match="slot 1600 out of range"):
         slots_module._slots(pool, list(range(most)) + [1600])
     assert slots_module._slots(pool, list(range(most)))[1] == "iekv_write_slots_cast_ids"
+
+
+def test_long_tables_are_uploaded_except_under_capture(monkeypatch):
+    """Tables of up to HOST_TABLE_MAX blocks ride in the launches' arguments; a longer one is
+    checked and uploaded, unless the stream is under capture, where nothing may be."""
+    uploads = []
+    monkeypatch.setattr(torch.cuda, "device", lambda device: nullcontext())
+    pool = SimpleNamespace(block_size=16, device=torch.device("cuda", 0),
+                           block_ids=lambda ids, what: uploads.append(len(ids)) or "uploaded")
+    most = slots_module.HOST_TABLE_MAX
+    for capturing in (False, True):
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+        for form in (list, tuple, np.array):
+            for blocks in (1, 512, most, most + 1, 4 * most):
+                del uploads[:]
+                table = form(list(range(blocks + 3)))
+                ids, fn = slots_module._context_table(pool, table, blocks * 16)
+                if blocks > most and not capturing:
+                    assert (ids, fn, uploads) == ("uploaded", "iekv_gather_rows_arrays", [blocks])
+                else:
+                    assert list(ids) == list(range(blocks)) and not uploads
+                    assert fn == "iekv_gather_rows_arrays_ids"
