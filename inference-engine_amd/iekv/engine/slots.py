@@ -84,17 +84,30 @@ def _rows(pool: KVPool, k: torch.Tensor, v: torch.Tensor):
     """K and V rows as the library reads them, and the types of the rows and the cache:
     contiguous rows in a wider type that it can round itself as they are, others cast
     first (the cast also makes them contiguous)."""
-    if k.dtype == v.dtype and (k.dtype, pool.dtype) in _CASTS and \
+    if k.dtype != pool.dtype and k.dtype == v.dtype and (k.dtype, pool.dtype) in _CASTS and \
             k.device == v.device == pool.device and not (k.is_neg() or v.is_neg()) and \
             k.is_contiguous() and v.is_contiguous():
         return k, v, _TYPES[k.dtype], _TYPES[pool.dtype]
-    return (k.to(device=pool.device, dtype=pool.dtype).contiguous(),
-            v.to(device=pool.device, dtype=pool.dtype).contiguous(),
-            _native.IEKV_TYPE_BYTES, _native.IEKV_TYPE_BYTES)
+    return (_in_cache_type(pool, k), _in_cache_type(pool, v), _native.IEKV_TYPE_BYTES,
+            _native.IEKV_TYPE_BYTES)
+
+
+def _in_cache_type(pool: KVPool, t: torch.Tensor) -> torch.Tensor:
+    return t.to(device=pool.device, dtype=pool.dtype).contiguous()
 
 
 def _write(pool: KVPool, first_layer: int, n_layers: int, n: int, k: torch.Tensor,
            v: torch.Tensor, slots) -> None:
+    if isinstance(slots, torch.Tensor) and k.dtype == pool.dtype:
+        # A step's writes of a model that computes in the cache's type: no more host work
+        # than the call needs.
+        where = slots.to(device=pool.device, dtype=torch.int64).contiguous()
+        kc, vc = _in_cache_type(pool, k), _in_cache_type(pool, v)
+        stride = kc.numel() // n_layers * kc.element_size() if n_layers > 1 else 0
+        _native.call("iekv_write_slots_layers", pool.native.handle, first_layer, n_layers,
+                     pool.block_size, kc.data_ptr(), vc.data_ptr(), stride, where.data_ptr(), n,
+                     current_stream_handle(pool.device))
+        return
     where, fn = _slots(pool, slots)
     kc, vc, row_type, cache_type = _rows(pool, k, v)
     stride = kc.numel() // n_layers * kc.element_size() if n_layers > 1 else 0
