@@ -209,8 +209,8 @@ enum {
  * float16, bfloat16 or e4m3; float16 or bfloat16 to e4m3; any other pair of different
  * types returns IEKV_ERR_INVALID): each element is rounded to nearest even on its way,
  * so no cast pass precedes the call. Row i of layer l is at k + l * layer_stride +
- * i * (row bytes in row_type). Values past the largest e4m3 value, and NaNs, become
- * NaN.
+ * i * (row bytes in row_type). To e4m3, magnitudes up to 464 round to at most 448, its
+ * largest value; larger ones, infinities and NaNs become NaN.
  * Replaces: `k.to(cache dtype)` and index_copy_ (ie/kernels/torch_backend.py:13-16). */
 int iekv_write_slots_cast(const iekv_pool* pool, int32_t first_layer, int32_t n_layers,
                           int32_t block_size, const void* k, const void* v,
@@ -480,8 +480,9 @@ int iekv_profile_stop(float* durations_ms, int32_t capacity, int32_t* count);
  * `status` is one device int32, overwritten with the IEKV_IDS_* bits of the
  * failed checks. Pools are compared by the memory they describe: two handles
  * over the same arrays count as one pool, and pools whose arrays overlap
- * otherwise are refused (IEKV_ERR_INVALID). Two or three small launches on `stream`, no host
- * synchronisation: the caller reads *status after the stream has passed them
+ * otherwise are refused (IEKV_ERR_INVALID). One small launch on `stream` for lists
+ * and destination pools within IEKV_CHECK_ONE_LAUNCH_IDS and _BLOCKS (the workspace
+ * is then not touched), else two or three; no host synchronisation: the caller reads *status after the stream has passed them
  * (and may skip the move, or read it after the move, to report). The launches
  * are not timed by iekv_profile_start. Calls that share a workspace or status
  * word must be ordered on one stream.
@@ -503,8 +504,12 @@ int iekv_check_ids(const iekv_pool* src, const int32_t* src_ids, const iekv_pool
  * them there, so a list that fails moves nothing. The call returns once the check's
  * result is known, in *bits (IEKV_IDS_*, 0 = the copy is on its way); `status` is a
  * word of pinned host memory the result arrives in, the caller's own until the call
- * returns. Lists or pools over the limits above return IEKV_ERR_CAPACITY, a stream
- * under capture IEKV_ERR_INVALID.
+ * returns. src_ids and dst_ids may be changed as soon as it has. The copy has only
+ * been enqueued, also where *bits is not 0 (it then moves nothing, but still reads
+ * its ids): leave `checked` and both pools alone until `stream` has passed the call,
+ * or change and free them in its order; other ids written to `checked` before that
+ * would be moved unchecked. Lists or pools over the limits above return
+ * IEKV_ERR_CAPACITY, a stream under capture IEKV_ERR_INVALID.
  * No counterpart in the reference (its copier checks no id). */
 int iekv_copy_direct_checked(const iekv_pool* src, const iekv_pool* dst, const int32_t* src_ids,
                              const int32_t* dst_ids, int32_t n_blocks, int32_t* checked,

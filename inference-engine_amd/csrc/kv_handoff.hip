@@ -243,7 +243,8 @@ struct RunOut {
   gptr<V> d;
   __amdgpu_buffer_rsrc_t run;
   __device__ __forceinline__ RunOut(gptr<V> at, int n) : d(at) {
-    // A run is at most a tile: kMaxTileBytes fits the resource.
+    // A run is a tile (at most kMaxTileBytes), a group of tiles (at most the chunk size) or
+    // a gather workgroup's vectors: its bytes fit the resource.
     if constexpr (kThrough)
       run = __builtin_amdgcn_make_buffer_rsrc((void*)at, 0, n * 16, kBufferWordFormat);
   }
@@ -551,9 +552,10 @@ struct InlineSlots {
 // What happens to a vector between its load and its store. Bytes<V> moves it; the
 // casts round each element to the cache's type, to nearest even, so rows computed in
 // a wider type are written without a cast pass (which reads the wide rows, writes the
-// narrow ones and is followed by a launch that reads them again). A float past the
-// largest e4m3 value becomes its NaN; NaNs become the cache type's canonical one, the
-// sign kept for e4m3: bit for bit what torch's casts give.
+// narrow ones and is followed by a launch that reads them again). Bit for bit what
+// torch's casts give: past 464, halfway from the largest e4m3 value (448) to the next
+// there would be, a value is e4m3's NaN; a NaN is bfloat16's canonical one, e4m3's with
+// its sign, and in float16 keeps its sign and the upper bits of its payload.
 template <typename V>
 struct Bytes {
   using Src = V;
@@ -869,7 +871,8 @@ ids_probe(const int32_t* __restrict__ ids, int32_t n, int64_t num_blocks,
 // then destinations, or -1 for every id when a check failed: a move that reads them
 // right behind on the stream then moves nothing (an id outside its pool is skipped),
 // so the host need not wait between the check and the move. *status may be pinned
-// host memory: it is written once, after the lists.
+// host memory: it is written once, by a thread that does not wait for the others' stores
+// to `checked`. Only the stream orders those, before the move that reads them.
 constexpr int kCheckThreads = 1024;
 constexpr int kCheckPerThread = 8;
 constexpr int32_t kCheckIds = kCheckThreads * kCheckPerThread;

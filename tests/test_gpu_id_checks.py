@@ -284,3 +284,97 @@ def test_checked_copies_around_the_one_launch_limits(gpu, n, blocks):
             dst.copy_blocks(dst, one(ids[:n]), one(np.roll(ids[n - 1:2 * n - 1], 1)))
         assert all(torch.equal(x, c) for x, c in zip(before, dst.k_caches))
         dst.copy_blocks(dst, one(ids[:n]), one(ids[n:]))
+
+
+@pytest.fixture
+def two_copiers(gpu):
+    from iekv.engine.copier import HipSlotCopier
+    from iekv.engine.pools import allocate_pool
+
+    def copier(seed):
+        k, v = allocate_pool(300, 2, 2, 1, 16, dtype=torch.uint8, device=gpu, zero=False)
+        k[0]._base.random_(0, 256, generator=torch.Generator(gpu).manual_seed(seed))
+        return HipSlotCopier(k, v, 2, check_device_ids=True)
+
+    return copier(11), copier(12)
+
+
+def slab(copier):
+    return copier.k_caches[0]._base
+
+
+def test_a_checked_copy_on_another_stream(gpu, two_copiers):
+    """copy_blocks(check_device_ids=True, stream=...) with valid and invalid lists in turn,
+    the stream busy: valid ones move, invalid ones raise and move nothing, and scratch
+    that is freed and taken again between the calls does not reach a copy in flight."""
+    src, dst = two_copiers
+    other = torch.cuda.Stream()
+    rng = np.random.default_rng(3)
+    busy = torch.randn(2048, 2048, device=gpu)
+    lists = []
+    for k in range(8):
+        s, d = rng.permutation(300)[:40], rng.permutation(300)[:40]
+        if k % 2:
+            d[7] = (d[8], 300)[k % 4 == 1]
+        lists.append([torch.from_numpy(x.astype(np.int32)).to(gpu) for x in (s, d)])
+    torch.cuda.synchronize()
+    want = slab(dst).view(2, 2, 300, 32).clone()
+    given = slab(src).view(2, 2, 300, 32)
+    for k, (s, d) in enumerate(lists):
+        with torch.cuda.stream(other):
+            for _ in range(4):
+                busy = busy @ busy * 1e-3
+        if k % 2:
+            with pytest.raises((IndexError, ValueError)):
+                dst.copy_blocks(src, s, d, stream=other)
+        else:
+            dst.copy_blocks(src, s, d, stream=other)
+            want[:, :, d.long()] = given[:, :, s.long()]
+        # the caller's own lists, and scratch of the same size, may be written at once
+        s.fill_(0)
+        d.fill_(1)
+        torch.full((80,), 5, dtype=torch.int32, device=gpu)
+    other.synchronize()
+    torch.cuda.synchronize()
+    assert torch.equal(slab(dst).view(2, 2, 300, 32), want)
+
+
+def test_a_checked_copy_refuses_pageable_words_and_captures(gpu, two_copiers):
+    """The result word has to be pinned host memory, and the call waits for the GPU, which a
+    stream under capture cannot: both are refused before anything is enqueued, and the
+    capture goes on."""
+    import ctypes
+
+    from iekv import _native
+
+    src, dst = two_copiers
+    s, d = (torch.arange(n, n + 9, dtype=torch.int32, device=gpu) for n in (0, 100))
+    checked = torch.empty(18, dtype=torch.int32, device=gpu)
+    pinned = torch.zeros(1, dtype=torch.int32).pin_memory()
+    bits = ctypes.c_int32()
+    before = slab(dst).clone()
+
+    def call(status):
+        _native.call("iekv_copy_direct_checked", src.pool.native.handle, dst.pool.native.handle,
+                     s.data_ptr(), d.data_ptr(), 9, checked.data_ptr(), status,
+                     torch.cuda.current_stream().cuda_stream, ctypes.byref(bits))
+
+    pageable = (ctypes.c_int32 * 1)()
+    with pytest.raises(_native.NativeError, match="not pinned host memory"):
+        call(ctypes.addressof(pageable))
+    graph = torch.cuda.CUDAGraph()
+    filled = torch.zeros(4, device=gpu)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        filled += 1
+        with pytest.raises(_native.NativeError, match="not under capture"):
+            call(pinned.data_ptr())
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+    assert filled.tolist() == [3.0] * 4 and torch.equal(slab(dst), before)
+    call(pinned.data_ptr())
+    torch.cuda.synchronize()
+    assert bits.value == 0
+    assert torch.equal(slab(dst).view(2, 2, 300, 32)[:, :, 100:109],
+                       slab(src).view(2, 2, 300, 32)[:, :, :9])

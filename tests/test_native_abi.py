@@ -688,3 +688,47 @@ def test_a_library_of_an_older_interface_is_refused_by_its_version(tmp_path):
                          timeout=300, env=dict(os.environ, IEKV_LIBRARY=str(library)))
     assert out.returncode == 0, out.stderr[-2000:]
     assert f"ABI version 21, expected {_native.ABI_VERSION}" in out.stdout
+
+
+def test_a_checked_copy_refuses_what_it_can_tell_before_any_launch(lib):
+    """iekv_copy_direct_checked without a GPU: a null result, pools of other shapes or
+    devices or that overlap, lists and pools over the one-launch limits (as their own
+    error, so that a caller can take the longer way), and missing or misaligned scratch;
+    an empty list is done at once, with no bits."""
+    from iekv import _native
+
+    a = _native.Pool([1 << 20, (1 << 20) + 64 * 16], tile_bytes=64, num_blocks=16, device=99)
+    b = _native.Pool([1 << 24, (1 << 24) + 64 * 16], tile_bytes=64, num_blocks=16, device=99)
+    wide = _native.Pool([1 << 24, (1 << 24) + 128 * 16], tile_bytes=128, num_blocks=16, device=99)
+    other = _native.Pool([1 << 28, (1 << 28) + 64 * 16], tile_bytes=64, num_blocks=16, device=1)
+    partial = _native.Pool([(1 << 20) + 64 * 8, 1 << 26], tile_bytes=64, num_blocks=16, device=99)
+    most = _native.CHECK_ONE_LAUNCH_BLOCKS
+    large = _native.Pool([1 << 32, 1 << 33], tile_bytes=64, num_blocks=most, device=99)
+    larger = _native.Pool([1 << 32, 1 << 33], tile_bytes=64, num_blocks=most + 1, device=99)
+    ids, checked, status = 1 << 12, 1 << 13, (ctypes.c_int32 * 2)()
+    word = ctypes.addressof(status)
+    bits = ctypes.c_int32(7)
+
+    def call(src, dst, n=2, checked=checked, status=word, out=ctypes.byref(bits)):
+        return lib.iekv_copy_direct_checked(src.handle, dst.handle, ids, ids, n, checked, status,
+                                            None, out)
+
+    def refused(code, expect, why):
+        assert code == expect, (code, lib.iekv_last_error())
+        assert why in lib.iekv_last_error().decode()
+
+    invalid, capacity = _native.IEKV_ERR_INVALID, _native.IEKV_ERR_CAPACITY
+    refused(call(a, b, out=None), invalid, "bits is null")
+    refused(call(a, wide), invalid, "differ in shape")
+    refused(call(a, other), invalid, "devices 99 and 1")
+    refused(call(a, partial), invalid, "overlap")
+    refused(call(a, b, n=-1), invalid, "negative")
+    refused(call(a, b, n=_native.CHECK_ONE_LAUNCH_IDS + 1), capacity, "8193 ids")
+    refused(call(a, larger), capacity, f"into {most + 1} blocks")
+    refused(call(a, b, checked=None), invalid, "null")
+    refused(call(a, b, status=None), invalid, "null")
+    refused(call(a, b, checked=checked + 2), invalid, "4-byte aligned")
+    refused(call(a, b, status=word + 1), invalid, "4-byte aligned")
+    for src, n in ((a, _native.CHECK_ONE_LAUNCH_IDS), (large, 2)):      # within the limits
+        refused(call(src, large, n=n), _native.IEKV_ERR_HIP, "device 99")
+    assert call(a, b, n=0, checked=None, status=None) == _native.IEKV_OK and bits.value == 0
