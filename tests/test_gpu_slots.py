@@ -498,3 +498,37 @@ def test_long_host_tables_gather_like_device_tables(gpu, blocks):
             gather_rows_arrays(pool, table[:-1].tolist() + [bad], blocks * 3)
     with pytest.raises(TypeError):
         gather_rows_arrays(pool, table[:-1].tolist() + [1.5], blocks * 3)
+
+
+@pytest.mark.parametrize("row_dtype,cache_dtype", [
+    (torch.float32, torch.float16), (torch.float32, torch.bfloat16),
+    (torch.float32, torch.float8_e4m3fn), (torch.float16, torch.float8_e4m3fn),
+    (torch.bfloat16, torch.float8_e4m3fn)], ids=str)
+def test_every_value_is_cast_as_torch_casts_it(gpu, row_dtype, cache_dtype):
+    """Every bit pattern of the row type, written as rows: the cache holds the bytes of
+    torch's cast on the GPU, ties, subnormals, overflow, infinities and NaNs of every
+    payload included. Rows aligned, and (the 16-bit types) one element in, which takes
+    the vectors at any address."""
+    from iekv.engine.slots import write_slots
+
+    bits = 8 * torch.tensor([], dtype=row_dtype).element_size()
+    dim, per_call = 1024, min(1 << 26, 1 << (bits - 1))
+    n = per_call // dim
+    k, v, pool = random_pool(n, 1, 1, dim, cache_dtype, gpu, layers=1, seed=1)
+    where = torch.arange(n, device=gpu)
+    whole = torch.int32 if bits == 32 else torch.int16
+    patterns = torch.arange(per_call, device=gpu, dtype=torch.int64)
+    for first in range(-(1 << (bits - 1)), 1 << (bits - 1), 2 * per_call):
+        rows = [(patterns + first + half * per_call).to(whole).view(row_dtype).view(n, 1, dim)
+                for half in (0, 1)]
+        write_slots(pool, 0, rows[0], rows[1], where)
+        for cache, row in zip(k + v, rows):
+            assert torch.equal(cache.view(torch.uint8),
+                               row.to(cache_dtype).view(torch.uint8)), first
+        if bits == 16:
+            for r in rows:
+                moved = torch.cat([r.reshape(-1)[:1], r.reshape(-1)])[1:].view(n, 1, dim)
+                assert moved.data_ptr() % 4
+                write_slots(pool, 0, moved, moved, where)
+                want = r.to(cache_dtype).view(torch.uint8)
+                assert all(torch.equal(c.view(torch.uint8), want) for c in k + v), first
