@@ -229,12 +229,13 @@ constexpr int kBufferWordFormat = 0x00020000;   // buffer resource word 3: 32-bi
 // smaller image when its reader comes or its buffer is written again, and the L2 has
 // nothing left to write back when the kernel ends. The stores go through a buffer
 // resource, the form in which the compiler lets the bit be chosen. Measured on MI355X,
-// non-temporal -> this: packs of 67 MB 25.9 -> 19.6 us, 126 MB 41.0 -> 38.5, 405 MB
-// and more level; a pack and its unpack 53.5 -> 41-47, 90 -> 76-84, 275 -> 235 us, of
-// 2.7 GB level; gathers of 126 MB 41.4 -> 32.7, 67 MB 25.4 -> 22.1, 1 GB level. With
-// the hint and the bit both nothing is gained. Ordinary stores packed 67 MB in 20.4 us
-// and 405 MB in 130 (126 with the hint). An unpack that writes its pool this way or
-// reads with ordinary loads loses part of it (405 MB pack and unpack 254 and 270 us).
+// three pools of each shape in turn, non-temporal -> this: packs into images of 34 MB
+// 13.2 -> 11.6 us, 67 MB 24.8 -> 21.1, 126 MB 39.8 -> 36.4, 405 MB 122 -> 116, 1.1 GB
+// 328 -> 317; a pack and its unpack 27.6 -> 24.5, 52.6 -> 50.2, 86.7 -> 73.3, 267 -> 232,
+// 720 -> 709 (the unpack alone reads an image that stayed in 36.7 us where it took 46, and one
+// that did not in 389 where it took 388); gathers of 20 MB 14.8 -> 12.7, 131 MB
+// 42.7 -> 40.1, 1 GB 315 -> 307. With the hint and the bit both nothing is gained; ordinary
+// stores pack 34 and 67 MB in 14.1 and 22.3, 405 MB in 121.
 constexpr int kImageStorePolicy = 16;   // sc1: device-coherent
 
 template <typename V, bool NT, bool IMAGE>
@@ -403,8 +404,9 @@ __device__ __forceinline__ void move_group(const PoolView& src, const PoolView& 
 // One list entry's share of a workgroup: chunk p of its tile in array a, or,
 // with group > 1, its tiles in arrays a * group .. a * group + group - 1. The
 // grouped path keeps at most 2 vectors per lane in flight: each one carries
-// its own source and destination address, and 4 were no faster (96-vector tiles
-// of 160 arrays 85.3 us against 85.2) while they took every launch that keeps 4
+// its own source and destination address, and 4 were no faster (1,024 blocks of 160
+// arrays of 128-vector tiles: direct 124.1 us against 124.6, pack and unpack 194.2 against
+// 194.3; 96-vector tiles 85.2 against 85.3) while they took every launch that keeps 4
 // or more in flight from 62 to 76 VGPRs.
 template <typename V, int U, bool NT, bool SRC_POOL, bool DST_POOL, bool HOST = false>
 __device__ __forceinline__ void move_unit(const PoolView& src, const PoolView& dst,
@@ -634,7 +636,7 @@ struct Cast {
 // takes any address: what rows cost is an access and a slot per lane, whatever the width.
 // Measured on MI355X, 3,001 rows of 2 KiB in 64 arrays at multiples of 8, 4, 2 and 1 bytes:
 // in vectors of that width 177, 198, 479 and 781 us (row by row, with one slot a row: 141,
-// 147, 294 and 469), in 16 bytes at any address 138, 137, 161 and 160. float32 rows at
+// 147, 294 and 469), in 16 bytes at any address 136, 135, 141 and 142. float32 rows at
 // multiples of 4, rounded to bfloat16: an element a lane 371, so 209 (cast by torch first 333);
 // bfloat16 rows of 500 elements to e4m3 244, so 67 (107).
 template <typename Op, int U, bool NT, bool LOOSE, typename Slots>
@@ -1636,10 +1638,10 @@ int check_write(const RowWrite& w, const int64_t* slots, int32_t n_tokens) {
 // Vectors per lane of a scatter workgroup with 16-byte source vectors: one, and four
 // where a cast leaves 4 bytes of each (float32 to e4m3), whose stores fill a quarter
 // of a cache line per wave and gain from being issued together. Measured on MI355X
-// with 1, 2 and 4 (us, XCD-grouped): 8B shape, 3,001 bfloat16 rows 127 / 145 / 137
-// (row by row: 146); the same rows from float32 202 / 204 / 212, 5.85 TB/s at 1 (cast
-// by torch first: 330); 70B share, 8,000 bfloat16 rows to e4m3 688 / 719 / 716 (torch
-// first: 1,083), 3,000 float32 rows to e4m3 477 / 442 / 404 (torch first: 580).
+// with 1, 2 and 4 (us, XCD-grouped): 8B shape, 3,001 bfloat16 rows 137 / 139 / 142
+// (row by row: 138-140); the same rows from float32 197 / 200 / 207, 6.0 TB/s at 1 (cast
+// by torch first: 330); 70B share, 8,000 bfloat16 rows to e4m3 691 / 722 / 718 (torch
+// first: 1,083), 3,000 float32 rows to e4m3 459 / 431 / 430 (torch first: 580).
 constexpr int kScatterU = 1;
 // Except launches of more workgroups than the GPU's 256 compute units hold at once (8 each)
 // and not quite twice as many: two vectors a lane leave no second, mostly empty turn. With
@@ -1651,11 +1653,11 @@ constexpr int64_t kScatterTwoLeast = 2049, kScatterTwoMost = 3584;
 template <typename Op>
 constexpr int kCastU = sizeof(typename Op::Dst) <= 4 ? 4 : 1;
 // The same for rows at addresses that are no multiple of their vectors (LOOSE), with 1, 2
-// and 4: 3,001 rows of 2,048 bytes at multiples of 8 138 / 139 / 145 us, at odd addresses
-// 160 / 144 / 156; 3,000 rows of 1,000 bytes in 56 arrays 60 / 61 / 67, of 162 13 / 13 / 13.
+// and 4: 3,001 rows of 2,048 bytes at multiples of 8 136 / 139 / 145 us, at odd addresses
+// 142 / 145 / 156; 3,000 rows of 1,000 bytes in 56 arrays 59 / 64 / 68, of 162 12 / 13 / 14.
 constexpr int kLooseU = 1;
 // And for rows of less than one vector (of 16 source bytes): 3,000 rows of 8 bytes in
-// 56 arrays, by random slots, 4.56 / 4.60 / 6.08, of 7 6.20 / 5.32 / 5.84.
+// 56 arrays, by random slots, 4.48 / 4.56 / 6.00, of 7 6.16 / 5.40 / 5.84.
 constexpr int kNarrowU = 2;
 // Slots one scatter launch carries in its arguments: a decode step's, and a longer
 // block (arguments cost the host per KiB, see InlineIds).
@@ -1771,11 +1773,10 @@ int launch_write(const RowWrite& w, SlotList list, int32_t n_tokens, hipStream_t
 }
 
 // Vectors per lane of a gather workgroup: 4 KiB of 16-byte vectors per workgroup.
-// Measured on MI355X with non-temporal stores (before RunOut's) and 1, 2 and 4: 8B
-// shape, 7,777 tokens 318 / 333 / 334 us
-// (6.41 TB/s at 1; row by row it took 354); 70B share, 8,000 tokens 418 / 444 / 413;
-// 1,000 tokens 43.6 / 44.0 / 45.6; 800-byte rows, 3,000 tokens 43.7 / 45.3 / 48.9.
-// XCD-grouped positions cost 3-12% everywhere at 1, so the gather keeps the plain
+// Measured on MI355X with 1, 2 and 4 (us): 8B shape, 7,777 tokens 307 / 352 / 356
+// (6.6 TB/s at 1; row by row 346); 70B share, 8,000 tokens 410 / 458 / 441; 1,000 tokens
+// 40.1 / 44.3 / 47.8; 800-byte rows, 3,000 tokens 41.9 / 45.0 / 50.4. XCD-grouped positions
+// cost 3-12% everywhere at 1 (with non-temporal stores), so the gather keeps the plain
 // order of staging-writing launches.
 constexpr int kGatherU = 1;
 // Table entries one gather launch carries in its arguments: a short block for the

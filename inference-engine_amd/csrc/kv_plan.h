@@ -124,9 +124,9 @@ inline int chunk_parts(int64_t tile_vecs, int vec_bytes, int64_t chunk_bytes) {
 // tile bytes tiles of one block in consecutive arrays (at most n_arrays), when
 // a tile's vector count divides the workgroup's lanes; 1 otherwise. Measured
 // on MI355X on one rank's share of the 70B-share workload at tp=8 (2 KiB
-// tiles, 160 arrays): two tiles per workgroup (4 KiB chunks) raised the
-// per-request direct copy from 4.17 to 5.76 TB/s and pack -> unpack from 4.34
-// to 6.15 TB/s; groups of 8 and 16 KiB were no faster.
+// tiles, 160 arrays), one tile, two, four and eight per workgroup: the per-request
+// direct copy 3.57 / 5.75 / 5.78 / 5.66 TB/s, pack -> unpack 3.89 / 6.59 / 6.53 /
+// 6.40, all requests in one launch 3.61 / 5.79 / 5.96 / 5.76.
 inline int tile_group(int64_t tile_vecs, int vec_bytes, int64_t chunk_bytes, int32_t n_arrays) {
   if (chunk_bytes <= 0 || tile_vecs * vec_bytes >= chunk_bytes || kThreads % tile_vecs) return 1;
   const int64_t group = chunk_bytes / (tile_vecs * vec_bytes);
