@@ -410,7 +410,12 @@ int iekv_noop(int32_t workgroups, int32_t launches, hipStream_t stream);
  *   nontemporal 1 for streaming (non-temporal) loads and stores, 0 for
  *               ordinary ones, -1 keeps the current setting; a pack that
  *               writes pinned host memory itself (a direct offload) uses
- *               ordinary ones for tiles of 16 KiB or more either way;
+ *               ordinary ones for tiles of 16 KiB or more either way; packs
+ *               into HBM and gathers write through instead of streaming
+ *               (their 16-byte vectors keep to the device-coherent level);
+ *               row writes that cast and rows or contexts that are no
+ *               multiples of 16 bytes always stream, moves of tiles that
+ *               are none never do;
  *   order       which (array, block) tiles are in flight together in the
  *               launches that write a pool (direct copy, unpack, restore):
  *               0 array-major (the 2L tiles of one block), 1 block-major
@@ -429,7 +434,10 @@ int iekv_noop(int32_t workgroups, int32_t launches, hipStream_t stream);
  *               in the order); a tile smaller than this whose 16-byte (or
  *               narrower) vectors divide 256 lanes is grouped instead: one
  *               workgroup moves a block's tiles in chunk_bytes / tile_bytes
- *               consecutive arrays; 0 moves one whole tile per workgroup; a
+ *               consecutive arrays; so is one of fewer than 256 vectors that
+ *               do not divide them, by as many arrays as keep its lanes busy
+ *               (up to 12 vectors when the launch reads pinned host memory,
+ *               40 when it writes it); 0 moves one whole tile per workgroup; a
  *               power of two from 64 to 1 MiB; -1 keeps the current setting.
  *               A launch that would exceed the dispatch limit of 2^32 - 1
  *               work-items halves the split, then spreads over several

@@ -983,27 +983,36 @@ using InlineKernel = void (*)(PoolView, PoolView, const char*, char*, InlineIds<
 // size W), empty for the other kernels.
 #define IEKV_EXTRA
 #define IEKV_PICK(KERNEL)                                                                       \
-  if (align >= 16) {                                                                            \
+  const int u = std::min(unroll, lane_vecs);                                                    \
+  if constexpr (SP && HP) {   /* streaming packs of 16-byte vectors only, see IEKV_PICK_HOST */ \
     *vec_bytes = 16;                                                                            \
-    const int u = std::min(unroll, lane_vecs);                                                  \
-    if (nt) {                                                                                   \
-      if (u >= 16) return KERNEL<u32x4, 16, true, SP, DP, HP IEKV_EXTRA>;                       \
-      if (u >= 8) return KERNEL<u32x4, 8, true, SP, DP, HP IEKV_EXTRA>;                         \
-      if (u >= 4) return KERNEL<u32x4, 4, true, SP, DP, HP IEKV_EXTRA>;                         \
-      if (u >= 2) return KERNEL<u32x4, 2, true, SP, DP, HP IEKV_EXTRA>;                         \
-      return KERNEL<u32x4, 1, true, SP, DP, HP IEKV_EXTRA>;                                     \
+    if (u >= 16) return KERNEL<u32x4, 16, true, SP, DP, HP IEKV_EXTRA>;                         \
+    if (u >= 8) return KERNEL<u32x4, 8, true, SP, DP, HP IEKV_EXTRA>;                           \
+    if (u >= 4) return KERNEL<u32x4, 4, true, SP, DP, HP IEKV_EXTRA>;                           \
+    if (u >= 2) return KERNEL<u32x4, 2, true, SP, DP, HP IEKV_EXTRA>;                           \
+    return KERNEL<u32x4, 1, true, SP, DP, HP IEKV_EXTRA>;                                       \
+  } else {                                                                                      \
+    if (align >= 16) {                                                                          \
+      *vec_bytes = 16;                                                                          \
+      if (nt) {                                                                                 \
+        if (u >= 16) return KERNEL<u32x4, 16, true, SP, DP, HP IEKV_EXTRA>;                     \
+        if (u >= 8) return KERNEL<u32x4, 8, true, SP, DP, HP IEKV_EXTRA>;                       \
+        if (u >= 4) return KERNEL<u32x4, 4, true, SP, DP, HP IEKV_EXTRA>;                       \
+        if (u >= 2) return KERNEL<u32x4, 2, true, SP, DP, HP IEKV_EXTRA>;                       \
+        return KERNEL<u32x4, 1, true, SP, DP, HP IEKV_EXTRA>;                                   \
+      }                                                                                         \
+      if (u >= 16) return KERNEL<u32x4, 16, false, SP, DP, HP IEKV_EXTRA>;                      \
+      if (u >= 8) return KERNEL<u32x4, 8, false, SP, DP, HP IEKV_EXTRA>;                        \
+      if (u >= 4) return KERNEL<u32x4, 4, false, SP, DP, HP IEKV_EXTRA>;                        \
+      if (u >= 2) return KERNEL<u32x4, 2, false, SP, DP, HP IEKV_EXTRA>;                        \
+      return KERNEL<u32x4, 1, false, SP, DP, HP IEKV_EXTRA>;                                    \
     }                                                                                           \
-    if (u >= 16) return KERNEL<u32x4, 16, false, SP, DP, HP IEKV_EXTRA>;                        \
-    if (u >= 8) return KERNEL<u32x4, 8, false, SP, DP, HP IEKV_EXTRA>;                          \
-    if (u >= 4) return KERNEL<u32x4, 4, false, SP, DP, HP IEKV_EXTRA>;                          \
-    if (u >= 2) return KERNEL<u32x4, 2, false, SP, DP, HP IEKV_EXTRA>;                          \
-    return KERNEL<u32x4, 1, false, SP, DP, HP IEKV_EXTRA>;                                      \
-  }                                                                                             \
-  if (align >= 8) { *vec_bytes = 8; return KERNEL<u32x2, 4, false, SP, DP, HP IEKV_EXTRA>; }    \
-  if (align >= 4) { *vec_bytes = 4; return KERNEL<uint32_t, 4, false, SP, DP, HP IEKV_EXTRA>; } \
-  if (align >= 2) { *vec_bytes = 2; return KERNEL<uint16_t, 4, false, SP, DP, HP IEKV_EXTRA>; } \
-  *vec_bytes = 1;                                                                               \
-  return KERNEL<uint8_t, 4, false, SP, DP, HP IEKV_EXTRA>;
+    *vec_bytes = align >= 8 ? 8 : align >= 4 ? 4 : align >= 2 ? 2 : 1;                          \
+    if (align >= 8) return KERNEL<u32x2, 4, false, SP, DP, HP IEKV_EXTRA>;                      \
+    if (align >= 4) return KERNEL<uint32_t, 4, false, SP, DP, HP IEKV_EXTRA>;                   \
+    if (align >= 2) return KERNEL<uint16_t, 4, false, SP, DP, HP IEKV_EXTRA>;                   \
+    return KERNEL<uint8_t, 4, false, SP, DP, HP IEKV_EXTRA>;                                    \
+  }
 
 template <bool SP, bool DP, bool HP>
 MoveKernel pick_kernel_as(int align, int unroll, int lane_vecs, bool nt, int* vec_bytes) {
@@ -1027,10 +1036,15 @@ InlineKernel<W> pick_inline_kernel_as(int align, int unroll, int lane_vecs, bool
 #undef IEKV_PICK
 
 // The kernels of a move; `host`: an unpack that reads pinned host memory, or a pack that
-// writes it (the HOST variants of move_entry and move_group).
+// writes it (the HOST variants of move_entry and move_group). Packs differ only where the
+// others write through: with streaming accesses of 16 bytes.
 #define IEKV_PICK_HOST(NAME)                                                                    \
-  if constexpr (SP != DP) {                                                                     \
+  if constexpr (!SP && DP) {                                                                    \
     if (host) return NAME##_as<SP, DP, true IEKV_EXTRA>(align, unroll, lane_vecs, nt, vec_bytes); \
+  }                                                                                             \
+  if constexpr (SP && !DP) {                                                                    \
+    if (host && nt && align >= 16)                                                              \
+      return NAME##_as<SP, DP, true IEKV_EXTRA>(align, unroll, lane_vecs, nt, vec_bytes);        \
   }                                                                                             \
   return NAME##_as<SP, DP, false IEKV_EXTRA>(align, unroll, lane_vecs, nt, vec_bytes);
 
@@ -1667,9 +1681,12 @@ constexpr int kLongSlots = IEKV_INLINE_IDS;
 // Launches a checked scatter whose rows are `row_elems` elements of Op (at least one
 // vector of them), in as many launches as the slots in the arguments (host slots), 32-bit
 // vector numbers and the dispatch limit need (iekv_plan::cut_rows).
+// Ordinary accesses (the non-temporal setting off) exist for aligned rows moved as bytes;
+// the other kinds always stream, so that the library holds half as many kernels of them.
 template <typename Op, int U, bool LOOSE = false>
 int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t row_elems,
                     hipStream_t stream) {
+  constexpr bool kOrdinary = std::is_same_v<Op, Bytes<u32x4>> && !LOOSE;
   const int64_t per_group = kThreads * U;
   const int32_t layers = w.pool->n_arrays / 2;
   const int64_t row_vecs = (row_elems + Op::kElems - 1) / Op::kElems;
@@ -1677,7 +1694,7 @@ int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t 
       row_vecs, w.n_layers, per_group, list.on_host ? kLongSlots : INT32_MAX, kMaxGrid / 2);
   DeviceGuard guard(w.pool->device);
   if (!guard.ok()) return guard.fail();
-  const bool nt = g_nontemporal.load() != 0;
+  [[maybe_unused]] const bool nt = g_nontemporal.load() != 0;
   const PoolView view = view_of(w.pool);
   const int64_t pool_rows = w.pool->num_blocks * w.block_size;
   // One launch: rows first .. first + n - 1 of layers l0 .. l0 + n_layers - 1 of the call.
@@ -1700,13 +1717,15 @@ int launch_write_as(const RowWrite& w, SlotList list, int32_t n_tokens, int64_t 
       constexpr int W = decltype(words)::value;
       InlineSlots<W> slots{};
       std::copy(list.slots + first, list.slots + first + n, slots.slots);
-      return nt ? go(kv_scatter_inline<Op, U, true, LOOSE, W>, slots)
-                : go(kv_scatter_inline<Op, U, false, LOOSE, W>, slots);
+      if constexpr (kOrdinary)
+        if (!nt) return go(kv_scatter_inline<Op, U, false, LOOSE, W>, slots);
+      return go(kv_scatter_inline<Op, U, true, LOOSE, W>, slots);
     };
     if (!list.on_host) {
       const DeviceSlots slots{list.slots + first};
-      return nt ? go(kv_scatter_rows<Op, U, true, LOOSE>, slots)
-                : go(kv_scatter_rows<Op, U, false, LOOSE>, slots);
+      if constexpr (kOrdinary)
+        if (!nt) return go(kv_scatter_rows<Op, U, false, LOOSE>, slots);
+      return go(kv_scatter_rows<Op, U, true, LOOSE>, slots);
     }
     return n <= kSmallSlots ? inlined(std::integral_constant<int, kSmallSlots>{})
                             : inlined(std::integral_constant<int, kLongSlots>{});
@@ -1809,12 +1828,15 @@ int check_gather(const iekv_pool* pool, int32_t first_array, int32_t n_arrays,
 }
 
 // One launch of a checked gather: `vecs` vectors of V per array, out of the blocks
-// of table[0 ..] (device memory, or `count` host ids for the arguments).
+// of table[0 ..] (device memory, or `count` host ids for the arguments). As in the scatter,
+// only aligned vectors of 16 bytes follow the non-temporal setting; narrow ones also always
+// find each lane's block.
 template <typename V, int U, bool LOOSE = false>
 int launch_gather_as(const iekv_pool* pool, int32_t first_array, GatherShape sh, IdList table,
                      int32_t count, char* out, int64_t out_stride, hipStream_t stream) {
-  const bool nt = g_nontemporal.load() != 0;
-  const bool spans = LOOSE || sh.tile_vecs % (kThreads * U) != 0;
+  constexpr bool kPlain = sizeof(V) == 16 && !LOOSE;
+  const bool nt = !kPlain || g_nontemporal.load() != 0;
+  const bool spans = !kPlain || sh.tile_vecs % (kThreads * U) != 0;
   const PoolView view = view_of(pool);
   const dim3 grid(static_cast<uint32_t>(sh.groups));
   auto inlined = [&](auto words) {
@@ -1824,10 +1846,12 @@ int launch_gather_as(const iekv_pool* pool, int32_t first_array, GatherShape sh,
     auto go = [&](auto kernel) {
       return dispatch(kernel, grid, stream, view, first_array, t, out, out_stride, sh);
     };
-    if (spans) return nt ? go(kv_gather_inline<V, U, true, true, LOOSE, W>)
-                         : go(kv_gather_inline<V, U, false, true, LOOSE, W>);
-    return nt ? go(kv_gather_inline<V, U, true, false, false, W>)
-              : go(kv_gather_inline<V, U, false, false, false, W>);
+    if constexpr (kPlain) {
+      if (!nt) return spans ? go(kv_gather_inline<V, U, false, true, false, W>)
+                            : go(kv_gather_inline<V, U, false, false, false, W>);
+      if (!spans) return go(kv_gather_inline<V, U, true, false, false, W>);
+    }
+    return go(kv_gather_inline<V, U, true, true, LOOSE, W>);
   };
   if (table.on_host)
     return count <= kSmallTable ? inlined(std::integral_constant<int, kSmallTable>{})
@@ -1836,10 +1860,12 @@ int launch_gather_as(const iekv_pool* pool, int32_t first_array, GatherShape sh,
   auto go = [&](auto kernel) {
     return dispatch(kernel, grid, stream, view, first_array, t, out, out_stride, sh);
   };
-  if (spans) return nt ? go(kv_gather_rows<V, U, true, true, LOOSE>)
-                       : go(kv_gather_rows<V, U, false, true, LOOSE>);
-  return nt ? go(kv_gather_rows<V, U, true, false, false>)
-            : go(kv_gather_rows<V, U, false, false, false>);
+  if constexpr (kPlain) {
+    if (!nt) return spans ? go(kv_gather_rows<V, U, false, true, false>)
+                          : go(kv_gather_rows<V, U, false, false, false>);
+    if (!spans) return go(kv_gather_rows<V, U, true, false, false>);
+  }
+  return go(kv_gather_rows<V, U, true, true, LOOSE>);
 }
 
 // A checked gather of context_len >= 1 rows of n_arrays arrays, in launches of as

@@ -532,3 +532,39 @@ def test_every_value_is_cast_as_torch_casts_it(gpu, row_dtype, cache_dtype):
                 write_slots(pool, 0, moved, moved, where)
                 want = r.to(cache_dtype).view(torch.uint8)
                 assert all(torch.equal(c.view(torch.uint8), want) for c in k + v), first
+
+
+def test_row_kernels_with_ordinary_accesses(gpu):
+    """The non-temporal setting off: aligned rows and contexts take ordinary accesses, the
+    other kinds go on streaming; the same bytes either way."""
+    from iekv import _native
+    from iekv.engine.slots import gather_rows_arrays, write_slots_layers
+
+    shape = _native.get_launch()
+    _native.set_launch(nontemporal=0)
+    try:
+        for dim, dtype, rows_dtype in ((128, torch.bfloat16, torch.bfloat16),
+                                       (81, torch.bfloat16, torch.bfloat16),
+                                       (3, torch.float16, torch.float16),
+                                       (128, torch.bfloat16, torch.float32)):
+            k, v, pool = random_pool(300, 16, 3, dim, dtype, gpu, layers=2, seed=dim)
+            n = 1600
+            rows = torch.randn(2, 2, n, 3, dim, device=gpu).to(rows_dtype)
+            slots = np.random.default_rng(dim).permutation(300 * 16)[:n].tolist()
+            where = torch.tensor(slots, device=gpu)
+            want = [c.clone().view(torch.int16) for c in k + v]
+            for l in range(2):
+                want[l][where] = rows[0, l].to(dtype).view(torch.int16)
+                want[2 + l][where] = rows[1, l].to(dtype).view(torch.int16)
+            write_slots_layers(pool, rows[0], rows[1], where)
+            write_slots_layers(pool, rows[0][:, :70].contiguous(), rows[1][:, :70].contiguous(),
+                               slots[:70])
+            assert all(torch.equal(w, c.view(torch.int16)) for w, c in zip(want, k + v)), dim
+            table = np.random.default_rng(dim + 1).permutation(300)[:90].tolist()
+            index = (torch.tensor(table, device=gpu)[:, None] * 16 +
+                     torch.arange(16, device=gpu)).reshape(-1)[:1437]
+            for form in (table, torch.tensor(table, dtype=torch.int32, device=gpu)):
+                got = gather_rows_arrays(pool, form, 1437).view(torch.int16)
+                assert all(torch.equal(g, w[index]) for g, w in zip(got, want)), dim
+    finally:
+        _native.set_launch(nontemporal=shape["nontemporal"])
