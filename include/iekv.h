@@ -490,10 +490,10 @@ int iekv_profile_stop(float* durations_ms, int32_t capacity, int32_t* count);
  * over the same arrays count as one pool, and pools whose arrays overlap
  * otherwise are refused (IEKV_ERR_INVALID). One small launch on `stream` for lists
  * and destination pools within IEKV_CHECK_ONE_LAUNCH_IDS and _BLOCKS (the workspace
- * is then not touched), else two or three; no host synchronisation: the caller reads *status after the stream has passed them
- * (and may skip the move, or read it after the move, to report). The launches
- * are not timed by iekv_profile_start. Calls that share a workspace or status
- * word must be ordered on one stream.
+ * is then not touched), else two or three; no host synchronisation: the caller
+ * reads *status after the stream has passed them (and may skip the move, or read
+ * it after the move, to report). The launches are not timed by iekv_profile_start.
+ * Calls that share a workspace or status word must be ordered on one stream.
  * No reference counterpart: the reference's copier slices its caches one block
  * at a time (ie/engine/copier.py:14-31) and checks no id; this gives callers
  * that keep ids on the device the checks the host-id calls make. */
